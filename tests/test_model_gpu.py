@@ -472,3 +472,37 @@ def test_random_config_sweep(case):
         first = m.prefill(cache, prompt)
         got = [first] + m.decode(cache, first, n_gen - 1)
     assert got == want
+
+
+@pytest.mark.parametrize("hidden,ff,vocab,t", [
+    (36, 20, 37, 4),       # 16-token tiles: rows and columns that fill no block or k-step
+    (2052, 36, 40, 16),    # ... with the deep batches of 2048 columns and more
+    (64, 1028, 300, 17),   # 32-token tiles, 15 tokens of the second block missing
+    (36, 4112, 2045, 251),  # gate/up on 2 x 2 blocks, the LM head on 2 x 4
+    (4108, 20, 300, 33),   # o and down products on 2 x 2 blocks, a 12-row last block
+    (36, 20, 2557, 251),   # the LM head on 5 x 2 blocks, a row count that is no multiple of 4
+])
+def test_products_of_several_tokens(hidden, ff, vocab, t):
+    """Every tile of the matrix-core products and their edges: all t rows of logits, alone
+    and after 3 cached tokens (fewer than the matrix cores take at this width), within 1e-4
+    of the CPU oracle (the bound for another summation order)."""
+    cfg = Config("llama", hidden, ff, 2, 2, 1, 16, vocab, rms_eps=1e-5, rope_theta=10000.0, tie_embeddings=True)
+    w = random_weights(cfg, seed=hidden + t, std=hidden ** -0.5)
+    rng = np.random.default_rng(hidden)
+    w["norm"] = (1 + 0.2 * rng.standard_normal(hidden)).astype(np.float32)
+    for lw in w["layers"]:
+        for k in ("attn_norm", "ffn_norm"):
+            lw[k] = (1 + 0.2 * rng.standard_normal(hidden)).astype(np.float32)
+    toks = [int(x) for x in random_prompt(t, t + 3, vocab)]
+    om = ol.OracleModel(cfg, w)
+    st = om.new_state(t + 3)
+    om.forward(st, toks[:3])
+    want = om.forward(st, toks[3:], all_logits=True)
+    alone = om.forward(om.new_state(t), toks[3:], all_logits=True)
+    with DeviceModel(cfg, w) as m:
+        cache = m.new_cache(t + 3)
+        m.forward(cache, toks[:3])
+        got = m.forward(cache, toks[3:], all_logits=True)
+        again = m.forward(m.new_cache(t), toks[3:], all_logits=True)
+    assert np.abs(got - want).max() < 1e-4
+    assert np.abs(again - alone).max() < 1e-4

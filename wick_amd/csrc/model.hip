@@ -6,9 +6,9 @@
 // Decode (t = 1) is HBM-bound: every weight is read once per token.  One wave
 // owns one output row, streams it with float4 loads (a wave reads 1 KiB of the
 // row per instruction) and reduces its 64 partial sums with a fixed butterfly,
-// so results are deterministic run to run.  For t > 1 each wave handles 4
-// tokens per weight pass (grid.y walks the token groups); the weight rows are
-// then re-read from L2 / MALL once per group.
+// so results are deterministic run to run.  2 or 3 tokens of a small model go
+// through one such weight pass together; more run on the matrix cores
+// (gemm_kernel).
 #include <hip/hip_runtime.h>
 
 #include <math.h>
@@ -320,131 +320,288 @@ __global__ __launch_bounds__(256) void gemv1_kernel(const GemvArgs a) {
     }
 }
 
-// Several tokens (prompt chunks): out rows of W . X^T on the f32 matrix cores.
-// A workgroup computes 16 output rows x 16*TB tokens as TB accumulators of
-// v_mfma_f32_16x16x4_f32 (A = 16 weight rows x 4 k, B = 4 k x 16 tokens); the
+// Several tokens: out rows of W . X^T on the f32 matrix cores
+// (v_mfma_f32_16x16x4_f32: A = 16 weight rows x 4 k, B = 4 k x 16 tokens).  The
 // contraction index is permuted so each lane loads whole float4s: MFMA e of
 // k-step s uses k = 16s + 4*(lane/16) + e for both operands.  Lane l then holds
-// rows row0 + 4*(l/16) + r of token tok0 + 16b + l%16.  The input rows are
-// already normalised (rmsnorm_kernel); the epilogues are gemv_kernel's.
+// rows row0 + 4*(l/16) + r of token tok0 + 16b + l%16.
+//
+// A workgroup computes one tile of 16*RB rows x 16*TB tokens; its NW waves deal
+// the k-steps out in batches of KU (wave w takes batches w, w + NW, ...: the
+// waves together read whole cache lines of every row) and their partial tiles
+// are summed through LDS in wave order.  The next batch's loads are in flight
+// during this one's products.
+//
+// What bounds it: chunks hold at most a few hundred tokens, so a CU's share of
+// the output is one small tile and every CU reads its rows and tokens at full
+// length from L2.  In the MFMA lane layout consecutive lanes are consecutive
+// rows, and the L1 then serves one lane (16 bytes) a cycle: 64 cache accesses
+// per load instruction counted, 13.5 bytes per cycle and CU whatever the tile.
+// So a wave loads each 16 x 16 block with 4 consecutive lanes on one row's 64
+// bytes (16 accesses) and passes it through its own piece of LDS.  256 tokens
+// of a 2048-wide layer (hidden 2048, FFN 5632): q/k/v 60 -> 27.6 us, o 22.5,
+// gate/up 194 -> 108, down 57 (o and down together 180 -> 80); without the
+// LDS turn 31, 27, 115, 69.  251 tokens at hidden 576, FFN 1536: 10.8 -> 5.8,
+// 6.2, 21.6 -> 14.7, 10.0 us.
 __device__ __forceinline__ f4 mfma4(float a, float b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
-template <int EPI, int TB>
-__global__ __launch_bounds__(256) void gemm_kernel(const GemvArgs a) {
-    // workgroup = one tile of 16 rows x 16*TB tokens; its 4 waves split k in
-    // four contiguous ranges and their partial tiles are summed through LDS
-    __shared__ f4 red[3][TB][2][64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int row0 = 16 * blockIdx.x;
-    const int tok0 = blockIdx.y * 16 * TB;
-    const int i = lane & 15, g = lane >> 4;
-    const float *wr = a.w + (size_t)min(row0 + i, a.rows - 1) * a.cols + 4 * g;
-    const float *w2r = EPI == kEpiSwiglu ? a.w2 + (size_t)min(row0 + i, a.rows - 1) * a.cols + 4 * g : wr;
-    const float *xr[TB];
-#pragma unroll
-    for (int b = 0; b < TB; b++) xr[b] = a.x + (size_t)min(tok0 + 16 * b + i, a.t - 1) * a.cols + 4 * g;
-    f4 acc[TB], acc2[TB];
-#pragma unroll
-    for (int b = 0; b < TB; b++) acc[b] = acc2[b] = f4{0.f, 0.f, 0.f, 0.f};
-    auto step = [&](const f4 &wv, const f4 &w2v, const f4 (&xv)[TB]) {
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-#pragma unroll
-            for (int b = 0; b < TB; b++) {
-                acc[b] = mfma4(wv[e], xv[b][e], acc[b]);
-                if (EPI == kEpiSwiglu) acc2[b] = mfma4(w2v[e], xv[b][e], acc2[b]);
-            }
-        }
-    };
-    // this wave's k range, in 16-wide steps
-    const int steps = a.cols / 16;
-    const int s0 = (w * steps) >> 2, s1 = ((w + 1) * steps) >> 2;
-    constexpr int KU = 4;  // steps per load batch: all of a batch's loads go out together
-    for (int st = s0; st < s1; st += KU) {
-        f4 wv[KU], w2v[KU], xv[KU][TB];
-#pragma unroll
-        for (int u = 0; u < KU; u++) {
-            const int k = 16 * min(st + u, s1 - 1);
-            wv[u] = *reinterpret_cast<const f4 *>(wr + k);
-            w2v[u] = wv[u];
-            if (EPI == kEpiSwiglu) w2v[u] = *reinterpret_cast<const f4 *>(w2r + k);
-#pragma unroll
-            for (int b = 0; b < TB; b++) xv[u][b] = *reinterpret_cast<const f4 *>(xr[b] + k);
-        }
-#pragma unroll
-        for (int u = 0; u < KU; u++)
-            if (st + u < s1) step(wv[u], w2v[u], xv[u]);
-    }
-    if (w > 0) {
-#pragma unroll
-        for (int b = 0; b < TB; b++) {
-            red[w - 1][b][0][lane] = acc[b];
-            if (EPI == kEpiSwiglu) red[w - 1][b][1][lane] = acc2[b];
-        }
-    }
-    __syncthreads();
-    if (w > 0) return;
-#pragma unroll
-    for (int b = 0; b < TB; b++) {
-#pragma unroll
-        for (int ww = 0; ww < 3; ww++) {
-            acc[b] += red[ww][b][0][lane];
-            if (EPI == kEpiSwiglu) acc2[b] += red[ww][b][1][lane];
-        }
-    }
-#pragma unroll
-    for (int b = 0; b < TB; b++) {
-        const int tok = tok0 + 16 * b + i;
-        if (tok >= a.t) continue;
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int row = row0 + 4 * g + r;
-            if (row >= a.rows) continue;
-            const float d = acc[b][r];
-            const size_t t = (size_t)tok;
-            if (EPI == kEpiStore) {
-                a.out0[t * a.ld0 + row] = d;
-            } else if (EPI == kEpiResid) {
-                a.out0[t * a.ld0 + row] += d;
-            } else if (EPI == kEpiQkv) {
-                if (row < a.split0)
-                    a.out0[t * a.ld0 + row] = d;
-                else if (row < a.split1)
-                    a.out1[t * a.ld1 + (row - a.split0)] = d;
-                else
-                    a.out2[t * a.ld2 + (row - a.split1)] = d;
-            } else {
-                a.out0[t * a.ld0 + row] = d / (1.0f + expf(-d)) * acc2[b][r];
-            }
-        }
-    }
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t gemm_rsrc(const float *base, unsigned bytes) {
+    const unsigned long long p = (unsigned long long)base;
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)p);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(p >> 32));
+    return __builtin_amdgcn_make_buffer_rsrc((void *)(((unsigned long long)hi << 32) | lo), (short)0,
+                                             (int)__builtin_amdgcn_readfirstlane(bytes), 0x00020000);
 }
 
-// rmsnorm (src/kernels.rs:343-349) of t rows of n floats: one workgroup per row,
-// a fixed-order reduction, xn = x * scale * g.
-__global__ __launch_bounds__(256) void rmsnorm_kernel(const float *__restrict__ x, const float *__restrict__ g,
-                                                      float eps, float *__restrict__ out, int n) {
-    __shared__ float red[4];
-    const float *xr = x + (size_t)blockIdx.x * n;
-    float ss = 0.0f;
-    for (int c = threadIdx.x; c < n; c += 256) ss = fmaf(xr[c], xr[c], ss);
-    ss = wave_sum(ss);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+__device__ __forceinline__ f4 gemm_load(__amdgpu_buffer_rsrc_t r, unsigned voff, unsigned soff) {
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    const u4 x = __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 0);
+    return f4{__uint_as_float(x[0]), __uint_as_float(x[1]), __uint_as_float(x[2]), __uint_as_float(x[3])};
+}
+
+template <int EPI, int RB, int TB, int NW, int KU>
+__global__ __launch_bounds__(64 * NW) void gemm_kernel(const GemvArgs a) {
+    constexpr int M = EPI == kEpiSwiglu ? 2 : 1;  // weight matrices
+    constexpr int NB = RB * TB;                   // 16 x 16 blocks of the tile
+    constexpr int NT = 16 * TB;                   // tokens of the tile
+    constexpr int PG = 64 * NW / NT;              // threads sharing a token's sum-of-squares parts
+    constexpr int BPW = (NB + NW - 1) / NW;       // blocks each wave finishes
+    constexpr int WL = 64 * (M * NB > KU * (M * RB + TB) ? M * NB : KU * (M * RB + TB));  // a wave's LDS, float4s
+    __shared__ f4 sm[NW][WL];
+    __shared__ float sss[PG][NT];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // Workgroup ids go round the 8 XCDs: all token tiles of a row tile run on
+    // one XCD, one after another, so its L2 reads each weight once.
+    const int nrt = (a.rows + 16 * RB - 1) / (16 * RB), ntt = (a.t + NT - 1) / NT;
+    const int slot = blockIdx.x >> 3;
+    const int rt = (blockIdx.x & 7) + 8 * (slot / ntt), tt = slot % ntt;
+    if (rt >= nrt) return;
+    const int row0 = 16 * RB * rt, tok0 = NT * tt;
+    const int i = lane & 15, g = lane >> 4;
+    // Rows and tokens past the end read as zero: within a 16-row block through
+    // the resource's bound, a whole block past it as block 0 (never stored).
+    // The k position is a lane's own offset, the row block a scalar one, so a
+    // batch costs one select per k-step: a k past the row reads out of bounds,
+    // as zero, without a branch (behind a branch the compiler waits for every
+    // load in flight, the next batch's too).
+    const unsigned pitch = (unsigned)a.cols * 4u;
+    const int wrows = min(16 * RB, a.rows - row0), toks = min(NT, a.t - tok0);
+    const __amdgpu_buffer_rsrc_t rw = gemm_rsrc(a.w + (size_t)row0 * a.cols, (unsigned)wrows * pitch);
+    const __amdgpu_buffer_rsrc_t rw2 =
+        M == 2 ? gemm_rsrc(a.w2 + (size_t)row0 * a.cols, (unsigned)wrows * pitch) : rw;
+    const __amdgpu_buffer_rsrc_t rx = gemm_rsrc(a.x + (size_t)tok0 * a.cols, (unsigned)toks * pitch);
+    unsigned so_w[RB], so_x[TB];
+#pragma unroll
+    for (int r = 0; r < RB; r++) so_w[r] = __builtin_amdgcn_readfirstlane(16 * r < wrows ? 16u * r * pitch : 0u);
+#pragma unroll
+    for (int t = 0; t < TB; t++) so_x[t] = __builtin_amdgcn_readfirstlane(16 * t < toks ? 16u * t * pitch : 0u);
+    // the row and 16-byte chunk this lane loads of each 16 x 16 block
+    const int lr = lane >> 2, lc = (lane & 3) ^ ((lr >> 1) & 3);
+    const unsigned vrow = (unsigned)lr * pitch + 16u * lc;
+
+    struct Batch {
+        f4 w[M][KU][RB], x[KU][TB];
+    };
+    auto load = [&](Batch &b, int n) {
+#pragma unroll
+        for (int u = 0; u < KU; u++) {
+            const int k = 16 * (KU * n + u);
+            const unsigned vo = k + 4 * lc < a.cols ? vrow + 4u * (unsigned)k : 0x80000000u;
+#pragma unroll
+            for (int r = 0; r < RB; r++) {
+                b.w[0][u][r] = gemm_load(rw, vo, so_w[r]);
+                if (M == 2) b.w[M - 1][u][r] = gemm_load(rw2, vo, so_w[r]);
+            }
+#pragma unroll
+            for (int t = 0; t < TB; t++) b.x[u][t] = gemm_load(rx, vo, so_x[t]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // through the wave's own LDS: stored as loaded, read in the product's lane
+    // layout (one wave's LDS operations run in order, so no barrier)
+    f4 *const mine = &sm[w][0];
+    const int rd = 4 * i + (g ^ ((i >> 1) & 3));
+    auto turn = [&](Batch &b) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int u = 0; u < KU; u++) {
+            f4 *q = mine + 64 * u * (M * RB + TB);
+#pragma unroll
+            for (int m = 0; m < M; m++)
+#pragma unroll
+                for (int r = 0; r < RB; r++) q[64 * (m * RB + r) + lane] = b.w[m][u][r];
+#pragma unroll
+            for (int t = 0; t < TB; t++) q[64 * (M * RB + t) + lane] = b.x[u][t];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    auto frags = [&](Batch &b) {
+#pragma unroll
+        for (int u = 0; u < KU; u++) {
+            const f4 *q = mine + 64 * u * (M * RB + TB) + rd;
+#pragma unroll
+            for (int m = 0; m < M; m++)
+#pragma unroll
+                for (int r = 0; r < RB; r++) b.w[m][u][r] = q[64 * (m * RB + r)];
+#pragma unroll
+            for (int t = 0; t < TB; t++) b.x[u][t] = q[64 * (M * RB + t)];
+        }
+    };
+    f4 acc[M][RB][TB];
+#pragma unroll
+    for (int m = 0; m < M; m++)
+#pragma unroll
+        for (int r = 0; r < RB; r++)
+#pragma unroll
+            for (int t = 0; t < TB; t++) acc[m][r][t] = f4{0.f, 0.f, 0.f, 0.f};
+    auto step = [&](const Batch &b) {
+#pragma unroll
+        for (int u = 0; u < KU; u++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int m = 0; m < M; m++)
+#pragma unroll
+                    for (int r = 0; r < RB; r++)
+#pragma unroll
+                        for (int t = 0; t < TB; t++) acc[m][r][t] = mfma4(b.w[m][u][r][e], b.x[u][t][e], acc[m][r][t]);
+    };
+
+    const int nbat = (a.cols + 16 * KU - 1) / (16 * KU), iters = (nbat + NW - 1) / NW;
+    Batch ba, bb;
+    load(ba, w);
+    // the values the epilogue needs, requested behind the first batch
+    f4 resid[EPI == kEpiResid ? BPW : 1];
+    if constexpr (EPI == kEpiResid) {
+#pragma unroll
+        for (int q = 0; q < BPW; q++) {
+            const int bl = min(w + NW * q, NB - 1);
+            const int tok = min(tok0 + 16 * (bl % TB) + i, a.t - 1), row = min(row0 + 16 * (bl / TB) + 4 * g, a.rows - 4);
+            resid[q] = *reinterpret_cast<const f4 *>(a.out0 + (size_t)tok * a.ld0 + row);
+        }
+    }
+    constexpr int SQ = 8;  // sum-of-squares parts a thread requests up front
+    const int pg = threadIdx.x / NT, ptk = threadIdx.x % NT;
+    const float *sp = a.ssq ? a.ssq + min(tok0 + ptk, a.t - 1) : nullptr;
+    float sq[SQ];
+    if (a.ssq) {
+#pragma unroll
+        for (int p = 0; p < SQ; p++) sq[p] = sp[(size_t)min(pg + p * PG, a.nssq - 1) * a.t];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    for (int it = 0; it < iters; it++) {
+        turn(ba);
+        load(ba, w + NW * (it + 1));
+        frags(bb);
+        step(bb);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int m = 0; m < M; m++)
+#pragma unroll
+        for (int r = 0; r < RB; r++)
+#pragma unroll
+            for (int t = 0; t < TB; t++) sm[w][64 * (m * NB + r * TB + t) + lane] = acc[m][r][t];
+    if (a.ssq) {
+        float ssum = 0.f;
+#pragma unroll
+        for (int p = 0; p < SQ; p++) ssum += pg + p * PG < a.nssq ? sq[p] : 0.f;
+        for (int p = pg + SQ * PG; p < a.nssq; p += PG) ssum += sp[(size_t)p * a.t];
+        sss[pg][ptk] = ssum;
+    }
     __syncthreads();
-    ss = (red[0] + red[1]) + (red[2] + red[3]);
-    const float scale = 1.0f / sqrtf(ss / (float)n + eps);
-    float *o = out + (size_t)blockIdx.x * n;
-    for (int c = threadIdx.x; c < n; c += 256) o[c] = xr[c] * scale * g[c];
+#pragma unroll
+    for (int q = 0; q < BPW; q++) {
+        const int bl = w + NW * q;
+        if (bl >= NB) break;
+        const int tk = 16 * (bl % TB) + i, tok = tok0 + tk, row = row0 + 16 * (bl / TB) + 4 * g;
+        f4 d[M];
+#pragma unroll
+        for (int m = 0; m < M; m++) {
+            d[m] = sm[0][64 * (m * NB + bl) + lane];
+#pragma unroll
+            for (int ww = 1; ww < NW; ww++) d[m] += sm[ww][64 * (m * NB + bl) + lane];
+        }
+        if (a.ssq) {
+            // rmsnorm's factor of the token (src/kernels.rs:343-349); its weight is in x
+            float ss = 0.f;
+#pragma unroll
+            for (int p = 0; p < PG; p++) ss += sss[p][tk];
+            const float scale = 1.0f / sqrtf(ss / (float)a.cols + a.eps);
+#pragma unroll
+            for (int m = 0; m < M; m++) d[m] *= scale;
+        }
+        const bool live = tok < a.t && row < a.rows;
+        const size_t tkn = (size_t)tok;
+        if constexpr (EPI == kEpiStore) {
+            if (live) {
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (row + r < a.rows) a.out0[tkn * a.ld0 + row + r] = d[0][r];
+            }
+        } else if constexpr (EPI == kEpiResid) {
+            const f4 x = resid[q] + d[0];
+            if (live) {
+                *reinterpret_cast<f4 *>(a.out0 + tkn * a.ld0 + row) = x;
+                if (a.xg) *reinterpret_cast<f4 *>(a.xg + tkn * a.ld0 + row) = x * *reinterpret_cast<const f4 *>(a.xnorm + row);
+            }
+            if (a.xg) {
+                // the block's share of the token's sum of squares, rows in order
+                float ss = live ? dot4(x, x, 0.f) : 0.f;
+                ss = rows_sum(ss);
+                const int part = row0 / 16 + bl / TB;
+                if (g == 0 && tok < a.t && 16 * part < a.rows) a.xssq[(size_t)part * a.t + tok] = ss;
+            }
+        } else if constexpr (EPI == kEpiQkv) {
+            // the splits are multiples of 16: a float4 lies in one output
+            if (live) {
+                float *o = row < a.split0   ? a.out0 + tkn * a.ld0 + row
+                           : row < a.split1 ? a.out1 + tkn * a.ld1 + (row - a.split0)
+                                            : a.out2 + tkn * a.ld2 + (row - a.split1);
+                *reinterpret_cast<f4 *>(o) = d[0];
+            }
+        } else {  // silu_mul: g / (1 + exp(-g)) * u
+            if (live) {
+                f4 h;
+#pragma unroll
+                for (int r = 0; r < 4; r++) h[r] = d[0][r] / (1.0f + expf(-d[0][r])) * d[M - 1][r];
+                *reinterpret_cast<f4 *>(a.out0 + tkn * a.ld0 + row) = h;
+            }
+        }
+    }
 }
 
 // step (graph-replayed decode loop): the token is tokens[*step + i].
+// xg: also x * xnorm (the first layer's norm weight) and the row's sum of
+// squares, for the products that apply the norm's factor (GemvArgs::ssq).
 __global__ __launch_bounds__(256) void embed_kernel(const float *__restrict__ embed, const uint32_t *__restrict__ tokens,
-                                                    const int *__restrict__ step, float *__restrict__ x, int hidden) {
+                                                    const int *__restrict__ step, float *__restrict__ x, int hidden,
+                                                    float *__restrict__ xg, const float *__restrict__ xnorm,
+                                                    float *__restrict__ xssq) {
+    __shared__ float red[4];
     const int i = blockIdx.x;
     const int at = (step ? *step : 0) + i;
     const f4 *src = reinterpret_cast<const f4 *>(embed + (size_t)tokens[at] * hidden);
     f4 *dst = reinterpret_cast<f4 *>(x + (size_t)i * hidden);
-    for (int c = threadIdx.x; c < hidden / 4; c += blockDim.x) dst[c] = src[c];
+    if (!xg) {
+        for (int c = threadIdx.x; c < hidden / 4; c += blockDim.x) dst[c] = src[c];
+        return;
+    }
+    f4 *dg = reinterpret_cast<f4 *>(xg + (size_t)i * hidden);
+    float ss = 0.0f;
+    for (int c = threadIdx.x; c < hidden / 4; c += blockDim.x) {
+        const f4 v = src[c];
+        dst[c] = v;
+        dg[c] = v * reinterpret_cast<const f4 *>(xnorm)[c];
+        ss = dot4(v, v, ss);
+    }
+    ss = wave_sum(ss);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    if (threadIdx.x == 0) xssq[i] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
 // sampler::argmax (src/sampler.rs:129-137): best = 0; for i: if x[i] > x[best]
@@ -648,31 +805,70 @@ hipError_t launch_gemv(int epi, const GemvArgs &a, hipStream_t s) {
     }
 }
 
-hipError_t launch_gemm(int epi, const GemvArgs &a, hipStream_t s) {
-    if (a.rows <= 0 || a.t <= 0) return hipSuccess;
-    if (a.cols % 16 != 0 || a.norm) return hipErrorInvalidValue;
-    constexpr int TB = 2;  // 32 tokens per workgroup tile
-    const dim3 grid((unsigned)((a.rows + 15) / 16), (unsigned)((a.t + 16 * TB - 1) / (16 * TB))), block(256);
-    switch (epi) {
-    case kEpiStore: hipLaunchKernelGGL((gemm_kernel<kEpiStore, TB>), grid, block, 0, s, a); break;
-    case kEpiResid: hipLaunchKernelGGL((gemm_kernel<kEpiResid, TB>), grid, block, 0, s, a); break;
-    case kEpiQkv: hipLaunchKernelGGL((gemm_kernel<kEpiQkv, TB>), grid, block, 0, s, a); break;
-    case kEpiSwiglu: hipLaunchKernelGGL((gemm_kernel<kEpiSwiglu, TB>), grid, block, 0, s, a); break;
-    default: return hipErrorInvalidValue;
-    }
+namespace {
+
+template <int EPI, int RB, int TB, int KU>
+hipError_t gemm_launch(const GemvArgs &a, hipStream_t s) {
+    constexpr int NW = 8;
+    const int nrt = (a.rows + 16 * RB - 1) / (16 * RB), ntt = (a.t + 16 * TB - 1) / (16 * TB);
+    hipLaunchKernelGGL((gemm_kernel<EPI, RB, TB, NW, KU>), dim3(8u * ((nrt + 7) / 8) * ntt), dim3(64 * NW), 0, s, a);
     return hipGetLastError();
 }
 
-hipError_t launch_rmsnorm(const float *x, const float *g, float eps, float *out, int t, int n, hipStream_t s) {
-    if (t <= 0) return hipSuccess;
-    hipLaunchKernelGGL(rmsnorm_kernel, dim3((unsigned)t), dim3(256), 0, s, x, g, eps, out, n);
-    return hipGetLastError();
+// What a tile of rb x tb blocks (of m weight matrices) costs: the products of
+// the busiest of the 256 CUs, each dearer the less the tile reuses what it
+// loads.  The model's order is the measured one where the tiles differ by more
+// than a few percent: 64 tokens at 2048 x 2048: 1x2 11.7 us, 2x2 15; 251
+// tokens at 2560 x 2048: 5x2 27.6, 2x2 32.4, 1x2 33+; at 2048 x 5632: 2x4 52.7,
+// 2x2 57; at 576 x 576: 1x2 and 2x2 6.2, 2x4 8.  (Gate/up on 2x4 blocks of both
+// matrices fills a CU's LDS with one workgroup: 113 us against 108 on 2x2.)
+double gemm_cost(const GemvArgs &a, int m, int rb, int tb) {
+    const long long wgs = (long long)((a.rows + 16 * rb - 1) / (16 * rb)) * ((a.t + 16 * tb - 1) / (16 * tb));
+    return (double)((wgs + 255) / 256) * (m * rb * tb + 0.5 * (m * rb + tb));
+}
+
+template <int EPI>
+hipError_t gemm_epi(const GemvArgs &a, hipStream_t s) {
+    constexpr int m = EPI == kEpiSwiglu ? 2 : 1;
+    if (a.t <= 16) {
+        // bound by the weights' arrival: more of them in flight per wave where a
+        // wave takes several batches (4 tokens, 2048 x 5632: 13.9 against 17.6
+        // us; at 576 columns a batch of 4 leaves waves idle, 4.3 against 3.6)
+        if constexpr (m == 1)
+            if (a.cols >= 2048) return gemm_launch<EPI, 1, 1, 4>(a, s);
+        return gemm_launch<EPI, 1, 1, 2>(a, s);
+    }
+    const int tiles[][2] = {{1, 2}, {2, 2}, {2, 4}, {5, 2}};
+    int best = 0;
+    for (int i = 1; i < (m == 2 ? 2 : 4); i++)
+        if (gemm_cost(a, m, tiles[i][0], tiles[i][1]) < gemm_cost(a, m, tiles[best][0], tiles[best][1])) best = i;
+    if constexpr (m == 1) {
+        if (best == 3) return gemm_launch<EPI, 5, 2, 1>(a, s);
+        if (best == 2) return gemm_launch<EPI, 2, 4, 1>(a, s);
+    }
+    return best == 1 ? gemm_launch<EPI, 2, 2, 1>(a, s) : gemm_launch<EPI, 1, 2, 1>(a, s);
+}
+
+}  // namespace
+
+hipError_t launch_gemm(int epi, const GemvArgs &a, hipStream_t s) {
+    if (a.rows <= 0 || a.t <= 0) return hipSuccess;
+    // 80 rows of a tile within a signed 32-bit byte range
+    if (a.cols % 4 != 0 || a.cols > (1 << 22) || a.norm) return hipErrorInvalidValue;
+    switch (epi) {
+    case kEpiStore: return gemm_epi<kEpiStore>(a, s);
+    case kEpiResid: return gemm_epi<kEpiResid>(a, s);
+    case kEpiQkv: return gemm_epi<kEpiQkv>(a, s);
+    case kEpiSwiglu: return gemm_epi<kEpiSwiglu>(a, s);
+    default: return hipErrorInvalidValue;
+    }
 }
 
 hipError_t launch_embed(const float *embed, const uint32_t *tokens, float *x, int t, int hidden, hipStream_t s,
-                        const int *step) {
+                        const int *step, float *xg, const float *xnorm, float *xssq) {
     if (t <= 0) return hipSuccess;
-    hipLaunchKernelGGL(embed_kernel, dim3((unsigned)t), dim3(256), 0, s, embed, tokens, step, x, hidden);
+    hipLaunchKernelGGL(embed_kernel, dim3((unsigned)t), dim3(256), 0, s, embed, tokens, step, x, hidden, xg, xnorm,
+                       xssq);
     return hipGetLastError();
 }
 

@@ -73,7 +73,7 @@ struct wick_hip_model {
     std::vector<void *> allocs;
     // activations, sized for `cap_t` tokens
     int cap_t = 0;
-    float *x = nullptr, *xn = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *att = nullptr, *h = nullptr;
+    float *x = nullptr, *xg = nullptr, *ssq = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *att = nullptr, *h = nullptr;
     // one token with the output projection fused into the decode kernel: the
     // per-unit partial products [units][hidden] and the residual after them
     float *oparts = nullptr, *xr = nullptr;
@@ -99,10 +99,10 @@ int upload(wick_hip_model *m, float **dst, const float *src, size_t n, const cha
 }
 
 void free_activations(wick_hip_model *m) {
-    void *bufs[] = {m->x, m->xn, m->q, m->k, m->v, m->att, m->h, m->oparts, m->xr};
+    void *bufs[] = {m->x, m->xg, m->ssq, m->q, m->k, m->v, m->att, m->h, m->oparts, m->xr};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
-    m->x = m->xn = m->q = m->k = m->v = m->att = m->h = m->oparts = m->xr = nullptr;
+    m->x = m->xg = m->ssq = m->q = m->k = m->v = m->att = m->h = m->oparts = m->xr = nullptr;
     m->cap_t = 0;
 }
 
@@ -114,7 +114,8 @@ int ensure_activations(wick_hip_model *m, int t) {
     struct {
         float **p;
         size_t n;
-    } want[] = {{&m->x, (size_t)c.hidden},  {&m->xn, (size_t)c.hidden}, {&m->q, (size_t)m->qd},
+    } want[] = {{&m->x, (size_t)c.hidden},  {&m->xg, (size_t)c.hidden}, {&m->q, (size_t)m->qd},
+                {&m->ssq, (size_t)(c.hidden + 15) / 16},
                 {&m->k, (size_t)m->kvd},    {&m->v, (size_t)m->kvd},    {&m->att, (size_t)m->qd},
                 {&m->h, (size_t)c.intermediate}};
     for (auto &w : want) {
@@ -180,26 +181,16 @@ int check_cache(const wick_hip_model *m, const wick_hip_kv *kv, int start, int t
     return WICK_HIP_OK;
 }
 
-// Prompt chunks of at least this many tokens run their products on the matrix
-// cores (gemm_kernel, after a separate RMSNorm pass); shorter ones stream the
-// weights through gemv_kernel, 4 tokens per pass.
-constexpr int kGemmMinTokens = 16;
+// Several tokens run their products on the matrix cores (gemm_kernel), except 2 or
+// 3 of a small model, which stream the weights through gemv_kernel in one pass:
+// the whole forward took 0.96 / 1.03 ms against 1.13 / 1.07 ms at hidden 576, but
+// 298 / 275 us against 259 / 235 us at hidden 2048.
+bool products_on_mfma(const wick_hip_model_config &c, int t) { return t >= 4 || (t > 1 && c.hidden > 1024); }
 
-// One product with a fused epilogue.  g.norm (optional) is the RMSNorm applied
-// to each input row: fused into the GEMV, or a separate pass into m->xn first.
-int product(wick_hip_model *m, int epi, wick::GemvArgs g, const char *what) {
-    hipError_t e;
-    if (g.t >= kGemmMinTokens && g.cols % 16 == 0) {
-        if (g.norm) {
-            if ((e = wick::launch_rmsnorm(g.x, g.norm, g.eps, m->xn, g.t, g.cols, m->stream)) != hipSuccess)
-                return hip_fail(e, "rmsnorm launch");
-            g.x = m->xn;
-            g.norm = nullptr;
-        }
-        e = wick::launch_gemm(epi, g, m->stream);
-    } else {
-        e = wick::launch_gemv(epi, g, m->stream);
-    }
+// One product with a fused epilogue: g.norm (optional) is the RMSNorm a GEMV
+// applies to its input rows; the GEMM takes it split (GemvArgs::ssq).
+int product(wick_hip_model *m, int epi, const wick::GemvArgs &g, bool gemm, const char *what) {
+    const hipError_t e = gemm ? wick::launch_gemm(epi, g, m->stream) : wick::launch_gemv(epi, g, m->stream);
     if (e != hipSuccess) return hip_fail(e, what);
     return WICK_HIP_OK;
 }
@@ -216,10 +207,35 @@ int forward_device(wick_hip_model *m, wick_hip_kv *kv, const uint32_t *tok_dev, 
     const hipStream_t s = m->stream;
     RC_TRY(ensure_activations(m, t));
     RC_TRY(ensure_logits(m, all_logits ? t : 1));
+    // gemm: each RMSNorm is split over two products -- whatever writes x (the
+    // embedding, the o and down products) also writes x * norm weight to xg and
+    // its sums of squares to ssq, and the product that reads xg applies the
+    // factor -- so no pass of its own reads x.
+    const bool gemm = products_on_mfma(c, t);
+    int nssq = 1;
     if (!embedded) {
-        hipError_t e = wick::launch_embed(m->embed, tok_dev, m->x, t, c.hidden, s, counters);
+        hipError_t e = wick::launch_embed(m->embed, tok_dev, m->x, t, c.hidden, s, counters, gemm ? m->xg : nullptr,
+                                          m->layers[0].attn_norm, m->ssq);
         if (e != hipSuccess) return hip_fail(e, "embed kernel launch");
     }
+    const auto normed = [&](wick::GemvArgs &g, const float *norm) {
+        g.eps = c.rms_eps;
+        if (gemm) {
+            g.x = m->xg;
+            g.ssq = m->ssq;
+            g.nssq = nssq;
+        } else {
+            g.x = m->x;
+            g.norm = norm;
+        }
+    };
+    const auto next_norm = [&](wick::GemvArgs &g, const float *norm) {
+        if (!gemm) return;
+        g.xg = m->xg;
+        g.xnorm = norm;
+        g.xssq = m->ssq;
+        nssq = (c.hidden + 15) / 16;
+    };
     // the gate/up product takes at most kMaxParts partial vectors of up to
     // 2048 floats (its input row in one pass)
     const int group = c.heads / c.kv_heads;
@@ -228,9 +244,7 @@ int forward_device(wick_hip_model *m, wick_hip_kv *kv, const uint32_t *tok_dev, 
     for (int li = 0; li < c.layers; li++) {
         const wick_hip_model::Layer &L = m->layers[li];
         wick::GemvArgs g{};
-        g.x = m->x;
-        g.norm = L.attn_norm;
-        g.eps = c.rms_eps;
+        normed(g, L.attn_norm);
         g.w = L.wqkv;
         g.out0 = m->q;
         g.out1 = m->k;
@@ -242,7 +256,7 @@ int forward_device(wick_hip_model *m, wick_hip_kv *kv, const uint32_t *tok_dev, 
         g.rows = m->qd + 2 * m->kvd;
         g.cols = c.hidden;
         g.t = t;
-        RC_TRY(product(m, wick::kEpiQkv, g, "qkv product launch"));
+        RC_TRY(product(m, wick::kEpiQkv, g, gemm, "qkv product launch"));
 
         // One token: attention and the output projection in one launch
         // (per-unit partial products), added to the residual by the gate/up
@@ -267,7 +281,7 @@ int forward_device(wick_hip_model *m, wick_hip_kv *kv, const uint32_t *tok_dev, 
             g.rows = c.intermediate;
             g.cols = c.hidden;
             g.t = 1;
-            RC_TRY(product(m, wick::kEpiSwiglu, g, "residual + gate/up product launch"));
+            RC_TRY(product(m, wick::kEpiSwiglu, g, false, "residual + gate/up product launch"));
 
             g = wick::GemvArgs{};
             g.x = m->h;
@@ -278,7 +292,7 @@ int forward_device(wick_hip_model *m, wick_hip_kv *kv, const uint32_t *tok_dev, 
             g.rows = c.hidden;
             g.cols = c.intermediate;
             g.t = 1;
-            RC_TRY(product(m, wick::kEpiResid, g, "down product launch"));
+            RC_TRY(product(m, wick::kEpiResid, g, false, "down product launch"));
             continue;
         }
 
@@ -292,12 +306,11 @@ int forward_device(wick_hip_model *m, wick_hip_kv *kv, const uint32_t *tok_dev, 
         g.rows = c.hidden;
         g.cols = m->qd;
         g.t = t;
-        RC_TRY(product(m, wick::kEpiResid, g, "o product launch"));
+        next_norm(g, L.ffn_norm);
+        RC_TRY(product(m, wick::kEpiResid, g, gemm, "o product launch"));
 
         g = wick::GemvArgs{};
-        g.x = m->x;
-        g.norm = L.ffn_norm;
-        g.eps = c.rms_eps;
+        normed(g, L.ffn_norm);
         g.w = L.w_gate;
         g.w2 = L.w_up;
         g.out0 = m->h;
@@ -305,7 +318,7 @@ int forward_device(wick_hip_model *m, wick_hip_kv *kv, const uint32_t *tok_dev, 
         g.rows = c.intermediate;
         g.cols = c.hidden;
         g.t = t;
-        RC_TRY(product(m, wick::kEpiSwiglu, g, "gate/up product launch"));
+        RC_TRY(product(m, wick::kEpiSwiglu, g, gemm, "gate/up product launch"));
 
         g = wick::GemvArgs{};
         g.x = m->h;
@@ -315,12 +328,17 @@ int forward_device(wick_hip_model *m, wick_hip_kv *kv, const uint32_t *tok_dev, 
         g.rows = c.hidden;
         g.cols = c.intermediate;
         g.t = t;
-        RC_TRY(product(m, wick::kEpiResid, g, "down product launch"));
+        next_norm(g, li + 1 < c.layers ? m->layers[li + 1].attn_norm : m->norm);
+        RC_TRY(product(m, wick::kEpiResid, g, gemm, "down product launch"));
     }
     wick::GemvArgs g{};
-    g.x = all_logits ? m->x : m->x + (size_t)(t - 1) * c.hidden;
-    g.norm = m->norm;
-    g.eps = c.rms_eps;
+    if (all_logits) {
+        normed(g, m->norm);
+    } else {
+        g.x = m->x + (size_t)(t - 1) * c.hidden;
+        g.norm = m->norm;
+        g.eps = c.rms_eps;
+    }
     g.w = m->lm_head;
     g.out0 = m->logits;
     g.ld0 = c.vocab;
@@ -328,10 +346,10 @@ int forward_device(wick_hip_model *m, wick_hip_kv *kv, const uint32_t *tok_dev, 
     g.cols = c.hidden;
     g.t = all_logits ? t : 1;
     if (all_logits) {
-        RC_TRY(product(m, wick::kEpiStore, g, "lm head product launch"));
+        RC_TRY(product(m, wick::kEpiStore, g, gemm, "lm head product launch"));
     } else {
         g.out1 = m->argparts;  // the first greedy step rides along with the product
-        RC_TRY(product(m, wick::kEpiArgmax, g, "lm head product launch"));
+        RC_TRY(product(m, wick::kEpiArgmax, g, false, "lm head product launch"));
     }
     return WICK_HIP_OK;
 }

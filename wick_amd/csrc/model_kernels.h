@@ -44,23 +44,31 @@ struct GemvArgs {
     float *xout;
     // kEpiResid: the value added to, resid[tok][row] (stride ld0); null: out0 itself
     const float *resid;
+    // launch_gemm: RMSNorm split over two products.  A kEpiResid product with
+    // xg also writes out0 * xnorm (the next norm's weight) to xg and, per token,
+    // each 16-row block's sum of squares to xssq[block][t]; the product that
+    // reads xg gets those sums as ssq (nssq blocks, added in order) and applies
+    // the norm's factor 1/sqrt(sum/cols + eps) to its own sums.
+    const float *ssq;
+    int nssq;
+    float *xg, *xssq;
+    const float *xnorm;
 };
 
 // out rows of a matrix-vector (or small matrix-matrix) product with the
 // epilogue `epi`; t tokens, cols % 4 == 0.
 hipError_t launch_gemv(int epi, const GemvArgs &a, hipStream_t s);
 
-// The same products for prompt chunks on the matrix cores: a.x holds normalised
-// rows (a.norm must be null), cols % 16 == 0.
+// The same products for several tokens on the matrix cores (a.norm must be
+// null, see GemvArgs::ssq; kEpiQkv: splits and rows multiples of 16).
 hipError_t launch_gemm(int epi, const GemvArgs &a, hipStream_t s);
-
-// out[i][:] = rmsnorm(x[i][:], g, eps) for i < t rows of n floats.
-hipError_t launch_rmsnorm(const float *x, const float *g, float eps, float *out, int t, int n, hipStream_t s);
 
 // x[i][:] = embed[tokens[i]][:] for i < t (token ids already validated).
 // step: when non-null, the token of row i is tokens[*step + i] (device counter).
+// xg: when non-null, also x[i][:] * xnorm and the row's sum of squares to xssq[i].
 hipError_t launch_embed(const float *embed, const uint32_t *tokens, float *x, int t, int hidden, hipStream_t s,
-                        const int *step = nullptr);
+                        const int *step = nullptr, float *xg = nullptr, const float *xnorm = nullptr,
+                        float *xssq = nullptr);
 
 // *out = sampler::argmax(x[0..n)) (first index of the maximum).
 // step, len: when non-null, the id goes to out[*step + 1] and both counters
