@@ -85,7 +85,9 @@ int wick_hip_attention_device(wick_hip_kv *kv, int layer, int heads, const float
  * handle's workspace: it needs kv_heads * ceil(group / 16) * 16 * 256 *
  * (head_dim + 2) floats, at most 8 Mi (e.g. up to 31 kv heads at head_dim 64
  * with group <= 16, or 15 at head_dim 128); a larger shape returns
- * WICK_HIP_EINVAL.  Prefill (t > 1) uses no workspace.  Every call on one GPU
+ * WICK_HIP_EINVAL.  Prefill (t > 1) uses no workspace: it never splits a few
+ * tokens' keys over workgroups, as wick_hip_attention_device does from the
+ * first call that may allocate.  Every call on one GPU
  * shares that array, so calls that overlap on one GPU (other handles or
  * streams included) race: serialise them.  Asynchronous on the handle's
  * stream. */
@@ -149,7 +151,7 @@ int wick_hip_kv_set_option(wick_hip_kv *kv, int option, int value);
 /* Number of workgroups the last attention call launched (for measurement). */
 int wick_hip_kv_last_grid(const wick_hip_kv *kv);
 
-/* Bytes of staging and decode workspace the handle has allocated so far, beyond
+/* Bytes of staging and attention workspace the handle has allocated so far, beyond
  * its K/V cache and RoPE / preparation tables (device and pinned host memory;
  * grown on demand by the allocating entry points, never by
  * wick_hip_attention_device_noalloc).  No counterpart in the reference: for

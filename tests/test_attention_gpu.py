@@ -510,3 +510,47 @@ def test_decode_hip_graph_replays_match_eager():
             s.synchronize()
             assert np.array_equal(att.cpu().numpy(), eager), f"replay {it}"
             kv.attention(it % layers, heads, qs[it % layers], L - 1)  # eager work between replays
+
+
+@pytest.mark.parametrize("t,start,heads,kv_heads,d", [
+    (2, 1000, 14, 2, 64),     # one block per kv head, most of it padding rows
+    (37, 12001, 14, 2, 64),   # 17 blocks, an uneven last one; uneven splits of an odd length
+    (20, 621, 9, 3, 64),      # the fewest steps that split
+    (16, 3000, 32, 8, 128),   # 4 heads per kv head, whole blocks
+    (3, 700, 6, 6, 128),      # one head per kv head, 3 rows
+    (64, 1984, 32, 4, 64),    # 128 blocks: the most that split
+    (2, 70000, 8, 1, 64),     # as many splits as states can be merged
+])
+def test_prefill_split_over_workgroups(t, start, heads, kv_heads, d):
+    """A few tokens over many keys: the blocks' keys shared by several workgroups and
+    merged, against the oracle and against the entry point that never splits; bit-stable;
+    and unsplit, without allocating, where the first call is captured into a graph."""
+    import torch
+    q, k, v = make_inputs(start, t, start, heads, kv_heads, d, theta=1e6)
+    blocks = kv_heads * ((t * heads // kv_heads + 15) // 16)
+    stream = torch.cuda.Stream()
+    qd = torch.from_numpy(q).cuda()
+    outs = [torch.full_like(qd, float("nan")) for _ in range(4)]
+    torch.cuda.synchronize()
+    with DeviceKvCache(1, start + t, kv_heads, d) as kv:
+        kv.append(0, 0, k, v)
+        kv.set_stream(stream.cuda_stream)
+        staged = kv.scratch_bytes()  # the append's
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            kv.attention_device(0, heads, qd.data_ptr(), t, start, outs[0].data_ptr())
+        assert kv.scratch_bytes() == staged and kv.last_grid() == blocks
+        for out in outs[1:3]:
+            kv.attention_device(0, heads, qd.data_ptr(), t, start, out.data_ptr())
+            assert kv.last_grid() > blocks and kv.last_grid() % blocks == 0
+        kv.attention_device_noalloc(0, heads, qd.data_ptr(), t, start, outs[3].data_ptr())
+        kv.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        captured, split, again, unsplit = (o.cpu().numpy() for o in outs)
+    assert np.array_equal(captured, unsplit)
+    assert np.array_equal(split, again)
+    want = ol.attention(q, k, v, t, start, heads, kv_heads, d)
+    ok, mabs, mrel = within_tol(split, want)
+    assert ok, (mabs, mrel)
+    assert within_tol(split, unsplit)[0]

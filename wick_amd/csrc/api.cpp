@@ -62,6 +62,9 @@ struct wick_hip_kv {
     // decode split-K workspace (partial softmax states of the chunks)
     float *part = nullptr;
     int ws_units = 0;
+    // split prefill workspace (kPrefillStates row states), made at first use and
+    // never moved
+    float *ppart = nullptr;
     // whether the static workspace's address was found on this device
     hipError_t static_rc = hipErrorNotInitialized;
     // options
@@ -220,6 +223,20 @@ int plan_decode(wick_hip_kv *kv, int layer, int group, int len, const float *q_d
     return WICK_HIP_OK;
 }
 
+// The split prefill's workspace; null where it cannot be had (the stream is
+// being captured and it is not there yet, or no memory): the call then runs
+// unsplit, which needs none.
+float *prefill_workspace(wick_hip_kv *kv) {
+    if (kv->ppart) return kv->ppart;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(kv->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) return nullptr;
+    if (hipMalloc(&kv->ppart, wick::kPrefillStates * (kv->head_dim + 2) * sizeof(float)) != hipSuccess) {
+        (void)hipGetLastError();
+        kv->ppart = nullptr;
+    }
+    return kv->ppart;
+}
+
 int run_attention(wick_hip_kv *kv, int layer, int heads, const float *q_dev, int t, int start, float *att_dev,
                   float *static_part = nullptr) {
     const int D = kv->head_dim;
@@ -259,6 +276,17 @@ int run_attention(wick_hip_kv *kv, int layer, int heads, const float *q_dev, int
                    ? 1
                    : 0;
     a.scale = scale;
+    a.splits = 1;
+    // (the no-allocation entry point never splits: its static workspace is one
+    // for all handles, and its prefill calls may overlap)
+    const int splits = static_part ? 1 : wick::prefill_splits(D, kv->num_cus, a);
+    if (splits > 1 && prefill_workspace(kv)) {
+        a.splits = splits;
+        a.rows32 = a.zigzag = 0;
+        a.po = kv->ppart;
+        a.pm = a.po + wick::kPrefillStates * D;
+        a.pl = a.pm + wick::kPrefillStates;
+    }
     kv->last_grid = wick::prefill_grid(D, a);
     hipError_t e = wick::launch_prefill(D, a, kv->stream);
     if (e != hipSuccess) return hip_fail(e, "prefill kernel launch");
@@ -496,7 +524,7 @@ int wick_hip_kv_create(int layers, int capacity, int kv_heads, int head_dim, wic
 void wick_hip_kv_destroy(wick_hip_kv *kv) {
     if (!kv) return;
     if (kv->stream) (void)hipStreamSynchronize(kv->stream);
-    float *bufs[] = {kv->k, kv->v, kv->q_dev, kv->att_dev, kv->kst_dev, kv->vst_dev, kv->part, kv->io_dev};
+    float *bufs[] = {kv->k, kv->v, kv->q_dev, kv->att_dev, kv->kst_dev, kv->vst_dev, kv->part, kv->ppart, kv->io_dev};
     for (float *b : bufs)
         if (b) (void)hipFree(b);
     if (kv->io_host) (void)hipHostFree(kv->io_host);
@@ -545,6 +573,7 @@ long long wick_hip_kv_scratch_bytes(const wick_hip_kv *kv) {
     if (!kv) return 0;
     size_t floats = kv->q_cap + kv->att_cap + 2 * kv->kst_cap + kv->io_cap + kv->io_host_cap;
     if (kv->part) floats += wick::decode_workspace_floats(kv->ws_units, kv->head_dim);
+    if (kv->ppart) floats += wick::kPrefillStates * (kv->head_dim + 2);
     return (long long)(floats * sizeof(float));
 }
 

@@ -35,6 +35,7 @@
 
 #include <math.h>
 
+#include <algorithm>
 #include <mutex>
 
 namespace wick {
@@ -1484,7 +1485,7 @@ constexpr long long lean_max_capacity() { return 0x7fffffffLL / (D * 4); }
 // is spread over as many MFMAs as at head_dim 128).  RB consecutive 16-row
 // blocks per workgroup: with two, every loaded tile serves both blocks (half
 // the tile loads per product), at 2 waves per SIMD.
-template <int D, int RB>
+template <int D, int RB, bool SPLIT = false>
 __device__ __forceinline__ void prefill_lean_body(const PrefillArgs &a) {
     using S = Shape<D>;
     static_assert(D == 64 || D == 128, "lean prefill: head_dim 64 or 128");
@@ -1496,7 +1497,8 @@ __device__ __forceinline__ void prefill_lean_body(const PrefillArgs &a) {
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kvh = blockIdx.x % a.kv_heads;
     const int nsb = (a.nblocks + RB - 1) / RB;
-    const int idx = (int)(blockIdx.x / a.kv_heads), half = (nsb + 1) >> 1;
+    const int bidx = (int)(blockIdx.x / a.kv_heads), half = (nsb + 1) >> 1;
+    const int idx = SPLIT ? bidx / a.splits : bidx, split = SPLIT ? bidx % a.splits : 0;
     const int sb = (a.zigzag && idx >= half) ? idx - half : nsb - 1 - idx;
     const float *Kh = a.k + (size_t)kvh * a.capacity * D;
     const float *Vh = a.v + (size_t)kvh * a.capacity * D;
@@ -1504,8 +1506,11 @@ __device__ __forceinline__ void prefill_lean_body(const PrefillArgs &a) {
     const int heads = a.kv_heads * a.group;
     const int nrows = a.t * a.group;
     const int kend = a.start + min(R * sb + R - 1, nrows - 1) / a.group + 1;
-    const int nt = (kend + 15) >> 4;
-    const int ks = 16 * ((w * nt) >> 2), ke = min(16 * (((w + 1) * nt) >> 2), kend);
+    // the workgroup's tiles t0 .. t0 + nt, a quarter to each wave
+    const int ntall = (kend + 15) >> 4;
+    const int t0 = SPLIT ? (int)((long long)split * ntall / a.splits) : 0;
+    const int nt = SPLIT ? (int)((long long)(split + 1) * ntall / a.splits) - t0 : ntall;
+    const int ks = 16 * (t0 + ((w * nt) >> 2)), ke = min(16 * (t0 + (((w + 1) * nt) >> 2)), kend);
 
     const float c = a.scale * kLog2e;
     f4 q[RB][S::KJ];
@@ -1567,8 +1572,10 @@ __device__ __forceinline__ void prefill_lean_body(const PrefillArgs &a) {
     }
     __syncthreads();
     // Merge the 4 waves' states (log2 units); wave 0 holds key 0, so M is
-    // finite.  The per-column weights, 1/sum and output row come first, once
-    // per column, so the per-element pass is 4 LDS float4 reads and FMAs.
+    // finite (a wave or split without keys keeps the finite floor and l = 0).
+    // The per-column weights, 1/sum and output row come first, once per column,
+    // so the per-element pass is 4 LDS float4 reads and FMAs.  A split's merged
+    // state goes to the workspace, unnormalised, at [row][split].
     if (threadIdx.x < R) {
         const int cc = threadIdx.x, rc = min(R * sb + cc, nrows - 1);
         float M = -INFINITY;
@@ -1581,9 +1588,19 @@ __device__ __forceinline__ void prefill_lean_body(const PrefillArgs &a) {
             sm_e[ww][cc] = e;
             L += sm_l[ww][cc] * e;
         }
-        sm_inv[cc] = 1.0f / L;
-        const int ic = rc / a.group, hc = rc % a.group;
-        sm_row[cc] = ic * heads + kvh * a.group + hc;
+        if constexpr (SPLIT) {
+            const int at = (kvh * nrows + rc) * a.splits + split;
+            sm_inv[cc] = 1.0f;
+            sm_row[cc] = at;
+            if (R * sb + cc < nrows) {
+                a.pm[at] = M;
+                a.pl[at] = L;
+            }
+        } else {
+            sm_inv[cc] = 1.0f / L;
+            const int ic = rc / a.group, hc = rc % a.group;
+            sm_row[cc] = ic * heads + kvh * a.group + hc;
+        }
     }
     __syncthreads();
     const int ncols = min(R, nrows - R * sb);
@@ -1592,7 +1609,7 @@ __device__ __forceinline__ void prefill_lean_body(const PrefillArgs &a) {
         f4 acc = *reinterpret_cast<const f4 *>(&sm_o[0][cc][d]) * sm_e[0][cc];
 #pragma unroll
         for (int ww = 1; ww < 4; ww++) acc += *reinterpret_cast<const f4 *>(&sm_o[ww][cc][d]) * sm_e[ww][cc];
-        *reinterpret_cast<f4 *>(a.att + (size_t)sm_row[cc] * D + d) = acc * sm_inv[cc];
+        *reinterpret_cast<f4 *>((SPLIT ? a.po : a.att) + (size_t)sm_row[cc] * D + d) = acc * sm_inv[cc];
     }
 }
 
@@ -1623,6 +1640,67 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void prefill_lean2_kernel_d64(
     const PrefillArgs a) {
     prefill_lean_body<64, 2>(a);
+}
+
+// A few rows over many keys (a short turn on a long kept prefix): the grid of
+// 16-row blocks leaves most CUs idle while each of its waves walks a quarter of
+// all keys, at about 1.35 us a step.  The key range is split again over
+// a.splits workgroups (prefill_splits), each writing its rows' states, and
+// prefill_merge_kernel, the next launch (3.5 us), combines them.  37 tokens on
+// 12001 positions, Qwen2.5 shape: 124 -> 26 us (34 workgroups -> 510); 5
+// tokens 124 -> 12; 16 on 8000, Llama-3-8B shape: 181 -> 34.  Two row blocks
+// per workgroup gain nothing here (29 us for the first).
+template <int D>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 128 ? 3 : 4)))
+void prefill_lean_split_kernel(const PrefillArgs a) {
+    prefill_lean_body<D, 1, true>(a);
+}
+
+// Workgroup = one row of [kv_heads][t * group].  Thread s owns split s's max and
+// sum; the row's D/4 float4s are summed by 256 / (D/4) groups of threads, each
+// over every such many splits, whose sums meet in LDS: one round trip for up
+// to 4 splits per group, a fixed order throughout.
+template <int D>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillArgs a) {
+    constexpr int C = D / 4, GR = 256 / C, U = 4;
+    __shared__ float se[kDecodeMaxChunks], sred[8];
+    __shared__ f4 so[GR][C];
+    const int tid = threadIdx.x, grp = tid / C, c = tid % C, w = tid >> 6;
+    const int row = blockIdx.x, S = a.splits;
+    const size_t base = (size_t)row * S;
+    const f4 *o = reinterpret_cast<const f4 *>(a.po + base * D) + c;
+    // clamped, in-bounds loads; the splits past S weigh 0
+    const int mine = min(tid, S - 1);
+    const float m = a.pm[base + mine], l = a.pl[base + mine];
+    f4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) v[u] = o[(size_t)min(grp + GR * u, S - 1) * C];
+    const float wm = wave_max(m);
+    if ((tid & 63) == 0) sred[w] = wm;
+    __syncthreads();
+    const float M = fmaxf(fmaxf(sred[0], sred[1]), fmaxf(sred[2], sred[3]));
+    const float e = tid < S ? exp2_fast(m - M) : 0.f;
+    se[tid] = e;
+    const float wl = wave_sum(tid < S ? l * e : 0.f);
+    if ((tid & 63) == 0) sred[4 + w] = wl;
+    __syncthreads();
+    f4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = grp; s0 < S; s0 += GR * U) {
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (s0 + GR * u < S) acc += v[u] * se[s0 + GR * u];
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = o[(size_t)min(s0 + GR * (U + u), S - 1) * C];
+    }
+    so[grp][c] = acc;
+    __syncthreads();
+    if (tid >= C) return;
+#pragma unroll
+    for (int k = 1; k < GR; k++) acc += so[k][c];
+    const float L = (sred[4] + sred[5]) + (sred[6] + sred[7]);
+    const int nrows = a.t * a.group, kvh = row / nrows, r = row % nrows;
+    const int head = (r / a.group) * (a.kv_heads * a.group) + kvh * a.group + r % a.group;
+    reinterpret_cast<f4 *>(a.att + (size_t)head * D)[c] = acc / L;
 }
 
 // ------------------------------------------------------------------ append
@@ -1874,12 +1952,42 @@ static bool prefill_uses_rows32(int head_dim, const PrefillArgs &a) {
 }
 
 int prefill_grid(int head_dim, const PrefillArgs &a) {
-    if (prefill_uses_rows32(head_dim, a)) return a.kv_heads * ((a.nblocks + 1) / 2);
-    return a.kv_heads * a.nblocks;
+    if (prefill_uses_rows32(head_dim, a)) return a.kv_heads * ((a.nblocks + 1) / 2) * a.splits;
+    return a.kv_heads * a.nblocks * a.splits;
+}
+
+int prefill_splits(int head_dim, int num_cus, const PrefillArgs &a) {
+    if (!prefill_has_rows32(head_dim, a.capacity)) return 1;
+    const int tg = head_dim == 128 ? Shape<128>::TG : Shape<64>::TG;
+    const long long units = (long long)a.kv_heads * a.nblocks;
+    const int steps = (a.start + a.t + 64 * tg - 1) / (64 * tg);  // of a wave of the last block, unsplit
+    // Where half the CUs or more have a workgroup a split gains little or loses
+    // (256 workgroups: 87 -> 107 us; 128: 46 -> 40), and below 6 steps the
+    // second launch costs what it saves (4 steps: 9.6 -> 10.3 us; 7: 12.6 ->
+    // 8.7).
+    if (2 * units > num_cus || steps < 6) return 1;
+    // One workgroup per CU; two where that leaves a wave more than 8 steps (34
+    // units of 94 steps: 27.6 -> 26.2 us; 32 of 63: 20.9, two 22.7).
+    long long s = num_cus / units;
+    if (steps > 8 * s) s = 2 * num_cus / units;
+    return (int)std::max(1LL, std::min({s, steps / 2LL, kPrefillSplitGrid / units, (long long)kDecodeMaxChunks}));
+}
+
+template <int D>
+static hipError_t launch_prefill_split(const PrefillArgs &a, int grid, hipStream_t s) {
+    hipLaunchKernelGGL(prefill_lean_split_kernel<D>, dim3(grid), dim3(256), 0, s, a);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(prefill_merge_kernel<D>, dim3((unsigned)(a.kv_heads * a.group * a.t)), dim3(256), 0, s, a);
+    return hipGetLastError();
 }
 
 hipError_t launch_prefill(int head_dim, const PrefillArgs &a, hipStream_t s) {
     const int grid = prefill_grid(head_dim, a);
+    if (a.splits > 1) {
+        if (!prefill_has_rows32(head_dim, a.capacity) || a.rows32 || !a.po) return hipErrorInvalidValue;
+        return head_dim == 128 ? launch_prefill_split<128>(a, grid, s) : launch_prefill_split<64>(a, grid, s);
+    }
     if (prefill_uses_rows32(head_dim, a) && head_dim == 128) {
         hipLaunchKernelGGL(prefill_lean2_kernel_d128, dim3(grid), dim3(256), 0, s, a);
     } else if (prefill_uses_rows32(head_dim, a)) {

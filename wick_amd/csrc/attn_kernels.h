@@ -74,8 +74,17 @@ struct PrefillArgs {
     int capacity, t, start, kv_heads, group, nblocks;
     int zigzag;       // the grid is resident at once; pair heavy and light blocks
     int rows32;       // lean kernels: two 16-row blocks per workgroup
+    int splits;       // lean kernels: workgroups sharing a block's keys (1: none)
     float scale;
+    // splits > 1: the states of row r of kv head h and split s, at
+    // [(h * t * group + r) * splits + s] (po: head_dim floats each)
+    float *po, *pm, *pl;
 };
+
+// Split prefill: most workgroups (of 16 rows) one launch has, so most row
+// states its workspace holds.
+constexpr int kPrefillSplitGrid = 512;
+constexpr size_t kPrefillStates = (size_t)kPrefillSplitGrid * kTileRows;
 
 struct AppendArgs {
     const float *ksrc, *vsrc;  // [t][kv_heads*D]
@@ -126,6 +135,9 @@ bool decode_interleaves(int head_dim, int group, int nchunks, int chunk);
 hipError_t launch_decode_oproj(int head_dim, DecodeArgs a, hipStream_t s);
 int prefill_grid(int head_dim, const PrefillArgs &a);
 hipError_t launch_prefill(int head_dim, const PrefillArgs &a, hipStream_t s);
+// How many workgroups share the keys of a block (PrefillArgs::splits) where the
+// workspace is there: 1 for most shapes.
+int prefill_splits(int head_dim, int num_cus, const PrefillArgs &a);
 hipError_t launch_append(int head_dim, const AppendArgs &a, hipStream_t s);
 // prep.hip: bias, QK-norm, RoPE of q and k; k and v appended to the cache.
 hipError_t launch_prep(int head_dim, const PrepArgs &a, hipStream_t s);
