@@ -31,6 +31,7 @@
 //       dmap(row, db) = 64*(db/4) + W*row + db%4 (W = min(D/16, 4)), so lane
 //       (i, g) loads V[p0+4g+m][64*seg + W*i .. +W) as one W-vector.
 #include "attn_kernels.h"
+#include "prep_row.h"
 #include "wave_ops.h"
 
 #include <math.h>
@@ -297,108 +298,6 @@ __device__ __forceinline__ void init_state(WaveState<D> &st) {
     st.l = 0.f;
 #pragma unroll
     for (int db = 0; db < Shape<D>::DB; db++) st.o[db] = f4{0.f, 0.f, 0.f, 0.f};
-}
-
-// ------------------------------------------------------------------ fused input preparation
-
-// The per-token preparation of src/model.rs:464-480 for one row of D floats,
-// bit-identical to wick's CPU arithmetic (and to prep_kernel): bias add;
-// rmsnorm_inplace (src/kernels.rs:351-357) -- a sequential f32 sum of squares
-// from -0.0, ss / D, 1 / sqrt(ss + eps) with IEEE divide and square root, then
-// (x * scale) * w; rope (src/model.rs:404-414) -- two rounded products and a
-// rounded sum per output, (sin, cos) from the host-filled table row.
-// 16 lanes own a row: lane l of the group holds the rotation quad j = 4l
-// (< D/2), i.e. elements j..j+3 and j+D/2..j+D/2+3, so all loads go out at
-// once; the sum of squares is carried through the lanes in element order by a
-// chain of shuffles (first half, then second half).  rowbase is the group's
-// first lane; every lane of the group must call this with the same row.
-// prep_load16 requests a row's inputs as one lane of its 16 holds them and
-// prep_finish16 does the arithmetic, so that a caller can request several
-// rows' inputs before it waits for any.
-struct PrepIn {
-    f4 u, w, bu, bw, nu, nw, c, sn;
-};
-
-template <int D>
-__device__ __forceinline__ PrepIn prep_load16(const float *src, const float *bias, const float *norm,
-                                              const float *cosr, const float *sinr, int l16) {
-    constexpr int H = D / 2, NQ = H / 4;
-    const int j = l16 < NQ ? 4 * l16 : 0;
-    PrepIn in;
-    in.u = *reinterpret_cast<const f4 *>(src + j);
-    in.w = *reinterpret_cast<const f4 *>(src + j + H);
-    in.bu = in.bw = in.nu = in.nw = in.c = in.sn = f4{0.f, 0.f, 0.f, 0.f};
-    if (bias) {
-        in.bu = *reinterpret_cast<const f4 *>(bias + j);
-        in.bw = *reinterpret_cast<const f4 *>(bias + j + H);
-    }
-    if (norm) {
-        in.nu = *reinterpret_cast<const f4 *>(norm + j);
-        in.nw = *reinterpret_cast<const f4 *>(norm + j + H);
-    }
-    if (cosr) {
-        in.c = *reinterpret_cast<const f4 *>(cosr + j);
-        in.sn = *reinterpret_cast<const f4 *>(sinr + j);
-    }
-    return in;
-}
-
-// The arithmetic of prep_row16 on loaded inputs; bias / norm / rot say which
-// steps apply (the pointers prep_load16 was given were non-null).
-template <int D>
-__device__ __forceinline__ void prep_finish16(PrepIn in, float *dst, bool bias, bool norm, float eps, bool rot,
-                                              int l16, int rowbase) {
-#pragma clang fp contract(off)
-    constexpr int H = D / 2, NQ = H / 4;
-    const bool mine = l16 < NQ;
-    const int j = mine ? 4 * l16 : 0;
-    f4 u = in.u, w = in.w;
-    if (bias) {
-        u = u + in.bu;
-        w = w + in.bw;
-    }
-    if (norm) {
-        float run = -0.0f;
-#pragma unroll
-        for (int i = 0; i < NQ; i++) {
-            float m = run;
-            m = m + u.x * u.x;
-            m = m + u.y * u.y;
-            m = m + u.z * u.z;
-            m = m + u.w * u.w;
-            run = __shfl(m, rowbase + i, 64);
-        }
-#pragma unroll
-        for (int i = 0; i < NQ; i++) {
-            float m = run;
-            m = m + w.x * w.x;
-            m = m + w.y * w.y;
-            m = m + w.z * w.z;
-            m = m + w.w * w.w;
-            run = __shfl(m, rowbase + i, 64);
-        }
-        run = run / (float)D;
-        const float scale = 1.0f / sqrtf(run + eps);
-        u = u * scale * in.nu;
-        w = w * scale * in.nw;
-    }
-    if (rot) {
-        const f4 a = u * in.c - w * in.sn;
-        const f4 b = w * in.c + u * in.sn;
-        u = a;
-        w = b;
-    }
-    if (mine) {
-        *reinterpret_cast<f4 *>(dst + j) = u;
-        *reinterpret_cast<f4 *>(dst + j + H) = w;
-    }
-}
-
-template <int D>
-__device__ __forceinline__ void prep_row16(const float *src, float *dst, const float *bias, const float *norm,
-                                           float eps, const float *cosr, const float *sinr, int l16, int rowbase) {
-    const PrepIn in = prep_load16<D>(src, bias, norm, cosr, sinr, l16);
-    prep_finish16<D>(in, dst, bias != nullptr, norm != nullptr, eps, cosr != nullptr, l16, rowbase);
 }
 
 // ------------------------------------------------------------------ lean building blocks

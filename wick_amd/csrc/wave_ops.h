@@ -15,6 +15,7 @@ namespace wick {
 
 constexpr int kDppQuadXor1 = 0xB1;       // quad_perm [1, 0, 3, 2]
 constexpr int kDppQuadXor2 = 0x4E;       // quad_perm [2, 3, 0, 1]
+constexpr int kDppRowShr1 = 0x111;       // lane i <- lane i - 1 within 16
 constexpr int kDppRowHalfMirror = 0x141;  // lane i <- lane 7 - i within 8
 constexpr int kDppRowMirror = 0x140;      // lane i <- lane 15 - i within 16
 
