@@ -95,6 +95,31 @@ def test_sampler_matches_oracle(vocab, name):
         assert ds.rng_state() == os_.rng.state()
 
 
+@pytest.mark.parametrize("vocab,top_k", [(4097, 2049), (4097, 0), (8192, 8191), (20001, 1025), (200003, 0)])
+def test_sort_over_many_workgroups(vocab, top_k):
+    """Candidate sets sorted by several workgroups: the fewest ids that take that path, whole
+    and ragged tiles, one id left out, the smallest top-k that does; with infinite, NaN
+    (both signs) and equal logits, sums that never reach top-p, and a temperature at which
+    most terms vanish."""
+    rng = np.random.default_rng(vocab + top_k)
+    for cfg in (SamplerConfig(temperature=0.9, top_k=top_k, top_p=0.9, seed=3),
+                SamplerConfig(temperature=0.05, top_k=top_k, top_p=1.0, min_p=1e-6, seed=4),
+                SamplerConfig(temperature=30.0, top_k=top_k, top_p=0.9999999, repetition_penalty=1.1, seed=5)):
+        with DeviceSampler(cfg, vocab) as ds:
+            os_ = ol.OracleSampler(cfg)
+            for kind in ("normal", "ties", "const", "-inf", "+inf", "-nan", "all -inf"):
+                x = logits_of("normal" if kind[-3:] in ("inf", "nan") else kind, vocab, rng)
+                at = rng.integers(0, vocab, 5)
+                if kind[-3:] in ("inf", "nan"):
+                    x[at] = {"+inf": np.inf, "-nan": np.float32(np.copysign(np.nan, -1.0))}.get(kind, -np.inf)
+                if kind == "all -inf":
+                    x[:] = -np.inf
+                history = rng.integers(0, vocab + 16, 100).astype(np.uint32)
+                with np.errstate(invalid="ignore"):
+                    check_draw(ds, os_, x, history, f"{vocab}/{top_k}/{cfg.temperature}/{kind}")
+            assert ds.rng_state() == os_.rng.state()
+
+
 def test_reference_unit_cases_on_device():
     """src/sampler.rs:150-171 through the device sampler."""
     logits = np.array([0.0, 3.0, 1.0, 2.9], np.float32)

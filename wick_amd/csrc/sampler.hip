@@ -2,7 +2,8 @@
 // kernels per draw, next to the logits the LM head wrote: a split kernel over
 // up to kSampleParts slices of the vocabulary (one workgroup streams only a
 // few tens of GB/s, so passes over the whole vocabulary are shared out), then
-// one workgroup that finishes the draw.
+// one workgroup that finishes the draw.  Larger candidate sets than the split
+// kernel's are sorted by many workgroups instead (launch_sorted).
 //
 // Phases (every branch that encloses a barrier depends only on kernel
 // arguments or on LDS values read after a barrier, so all threads take it):
@@ -31,6 +32,7 @@
 
 #include "exp_f32.h"
 #include "sampler_kernels.h"
+#include "wave_ops.h"
 
 namespace wick {
 namespace {
@@ -728,7 +730,455 @@ __global__ __launch_bounds__(kT) void sample_kernel(SampleArgs a) {
     }
 }
 
+// ---------------------------------------------------------------- large candidate sets
+//
+// Thousands of candidates or all ids (sorts_vocabulary).  One workgroup took
+// 2.3 ms a draw over all of 151936 ids: it sorted them at a few tens of GB/s
+// and added the probabilities one at a time.  Here the whole vocabulary is sorted by a
+// stable radix sort over as many workgroups as it fills, and the three walks in
+// wick's order take thousands of terms at once where that gives the same bits
+// (walk): 100 us a draw in 9 launches, each bound by its own latency (under the
+// profiler: histograms 5-6 us, moves 12-14, sum 16, draw 23).
+//
+// Radix sort, 11 + 11 + 10 bits: per pass a histogram of every tile of kTile
+// entries (sort_hist_kernel), then every tile finds its digits' places from all
+// tiles' histograms and moves its entries (sort_move_kernel).  A wave owns 256
+// consecutive entries of the tile and ranks equal digits by ballots, so the
+// order among them is kept.  The first pass reads the logits, the last leaves
+// the candidates' ids and exp terms.
+
+constexpr int kSortE = 4, kTile = kT * kSortE;
+static_assert(kTile == kSampleTile, "the sampler's buffers hold one histogram per tile");
+
+// the lanes of this wave with the same BITS-bit digit
+template <int BITS>
+__device__ __forceinline__ unsigned long long same_digit(uint32_t d, bool valid) {
+    unsigned long long peers = __ballot(valid);
+#pragma unroll
+    for (int b = 0; b < BITS; b++) {
+        const bool bit = (d >> b) & 1u;
+        const unsigned long long m = __ballot(bit);
+        peers &= bit ? m : ~m;
+    }
+    return peers;
+}
+
+__device__ __forceinline__ int tile_entry(int e) {
+    return (int)blockIdx.x * kTile + (int)(threadIdx.x >> 6) * 64 * kSortE + 64 * e + (int)(threadIdx.x & 63);
+}
+
+// PASS 0 takes key bits 0..10, PASS 1 bits 11..21, PASS 2 bits 22..31.
+template <int PASS>
+__global__ __launch_bounds__(kT) void sort_hist_kernel(SampleArgs a) {
+    constexpr int BITS = PASS < 2 ? 11 : 10, NB = 1 << BITS, SHIFT = 11 * PASS;
+    __shared__ uint32_t cnt[NB];
+    __shared__ uint32_t least[kW];
+    const uint2 *src = reinterpret_cast<const uint2 *>(PASS == 1 ? a.key0 : a.key1);
+    uint32_t key[kSortE], best = 0xffffffffu;
+#pragma unroll
+    for (int e = 0; e < kSortE; e++) {
+        const int i = min(tile_entry(e), a.vocab - 1);
+        key[e] = PASS == 0 ? desc_key(a.logits[i]) : src[i].x;
+        best = min(best, key[e]);
+    }
+    for (int b = threadIdx.x; b < NB; b += kT) cnt[b] = 0u;
+    if (PASS == 0) {
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) best = min(best, (uint32_t)__shfl_xor((int)best, off, 64));
+        if ((threadIdx.x & 63) == 0) least[threadIdx.x >> 6] = best;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < kSortE; e++) {
+        const bool valid = tile_entry(e) < a.vocab;
+        const uint32_t d = (key[e] >> SHIFT) & (NB - 1);
+        const unsigned long long peers = same_digit<BITS>(d, valid);
+        if (valid && (peers & ((1ull << (threadIdx.x & 63)) - 1ull)) == 0ull) atomicAdd(&cnt[d], (uint32_t)__popcll(peers));
+    }
+    __syncthreads();
+    for (int b = threadIdx.x; b < NB; b += kT) a.tile_hist[(size_t)blockIdx.x * NB + b] = (uint16_t)cnt[b];
+    if (PASS == 0 && threadIdx.x == 0) {
+        for (int j = 1; j < kW; j++) best = min(best, least[j]);
+        a.tile_least[blockIdx.x] = best;
+    }
+}
+
+template <int PASS>
+__global__ __launch_bounds__(kT) void sort_move_kernel(SampleArgs a) {
+    constexpr int BITS = PASS < 2 ? 11 : 10, NB = 1 << BITS, SHIFT = 11 * PASS, U = 16;
+    __shared__ __attribute__((aligned(16))) uint16_t wcnt[kW][NB];  // a wave's digit counts, then its places within the tile's
+    __shared__ uint32_t base[NB];
+    __shared__ uint32_t wsum[kW];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, tiles = gridDim.x;
+    const uint2 *src = reinterpret_cast<const uint2 *>(PASS == 1 ? a.key0 : a.key1);
+    uint32_t key[kSortE], id[kSortE], pos[kSortE];
+#pragma unroll
+    for (int e = 0; e < kSortE; e++) {
+        const int i = min(tile_entry(e), a.vocab - 1);
+        const uint2 in = PASS == 0 ? make_uint2(desc_key(a.logits[i]), (uint32_t)i) : src[i];
+        key[e] = in.x;
+        id[e] = in.y;
+    }
+    // the thread's two bins over all tiles, and over the tiles before this one
+    const bool owner = 2 * tid < NB;
+    uint32_t tot0 = 0u, tot1 = 0u, bef0 = 0u, bef1 = 0u;
+    if (owner) {
+        // 16-bit counts: every tile reads all of them, 27 GB/s a CU
+        const uint32_t *h = reinterpret_cast<const uint32_t *>(a.tile_hist) + tid;
+        for (int t0 = 0; t0 < tiles; t0 += U) {
+            uint32_t c[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) c[u] = h[(size_t)min(t0 + u, tiles - 1) * (NB / 2)];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                c[u] = t0 + u < tiles ? c[u] : 0u;
+                if (t0 + u == (int)blockIdx.x) {
+                    bef0 = tot0;
+                    bef1 = tot1;
+                }
+                tot0 += c[u] & 0xffffu;
+                tot1 += c[u] >> 16;
+            }
+        }
+    }
+    for (int b = tid; b < kW * NB / 2; b += kT) reinterpret_cast<uint32_t *>(&wcnt[0][0])[b] = 0u;
+    // exclusive prefix of the bins' totals over the threads
+    uint32_t inc = tot0 + tot1;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t t = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += t;
+    }
+    if (lane == 63) wsum[w] = inc;
+    __syncthreads();
+    uint32_t excl = inc - tot0 - tot1;
+#pragma unroll
+    for (int j = 0; j < kW; j++) excl += j < w ? wsum[j] : 0u;
+    if (owner) {
+        base[2 * tid] = excl + bef0;
+        base[2 * tid + 1] = excl + tot0 + bef1;
+    }
+#pragma unroll
+    for (int e = 0; e < kSortE; e++) {
+        const bool valid = tile_entry(e) < a.vocab;
+        const uint32_t d = (key[e] >> SHIFT) & (NB - 1);
+        const unsigned long long peers = same_digit<BITS>(d, valid);
+        const uint32_t rank = (uint32_t)__popcll(peers & ((1ull << lane) - 1ull)), before = wcnt[w][d];
+        pos[e] = before + rank;
+        __builtin_amdgcn_wave_barrier();
+        if (valid && rank == 0u) wcnt[w][d] = (uint16_t)(before + (uint32_t)__popcll(peers));
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    // a wave's counts become its places among the tile's (two 16-bit bins at a
+    // time: none passes kTile)
+    if (owner) {
+        uint32_t c[kW], off = 0u;
+#pragma unroll
+        for (int j = 0; j < kW; j++) c[j] = *reinterpret_cast<const uint32_t *>(&wcnt[j][2 * tid]);
+#pragma unroll
+        for (int j = 0; j < kW; j++) {
+            *reinterpret_cast<uint32_t *>(&wcnt[j][2 * tid]) = off;
+            off += c[j];
+        }
+    }
+    float mx = 0.0f;
+    if (PASS == 2) {
+        uint32_t best = 0xffffffffu;
+        for (int t = lane; t < tiles; t += 64) best = min(best, a.tile_least[t]);
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) best = min(best, (uint32_t)__shfl_xor((int)best, o, 64));
+        mx = key_value(best);
+    }
+    __syncthreads();
+    const uint32_t k = top_k_of(a);
+#pragma unroll
+    for (int e = 0; e < kSortE; e++) {
+        if (tile_entry(e) >= a.vocab) continue;
+        const uint32_t d = (key[e] >> SHIFT) & (NB - 1), to = base[d] + wcnt[w][d] + pos[e];
+        if (PASS == 2) {
+            // src/sampler.rs:95-98, the terms before their sum
+            if (to < k) {
+                a.res_idx[to] = id[e];
+                a.res_prob[to] = exp_f32((key_value(key[e]) - mx) / a.temperature);
+            }
+        } else if (to < (uint32_t)a.vocab) {
+            reinterpret_cast<uint2 *>(PASS == 0 ? a.key0 : a.key1)[to] = make_uint2(key[e], id[e]);
+        }
+    }
+}
+
+// wick's running f32 sums, term by term in order, by the whole workgroup:
+//   kWalkSum   acc + p[0] + p[1] + ...
+//   kWalkReach the same until the sum reaches limit (>=): *hit is that term
+//   kWalkDrain acc - p[0] - p[1] - ... until it is <= 0: *hit is that term
+// (*hit = -1 where it never does), the value there or at the end returned in
+// every thread.  No NaNs; p >= 0 and never grows by more than a rounding.
+//
+// While acc stays within one power of two, acc = R u with u its ulp and R an
+// integer, acc + p rounds to (R + rint(p/u)) u -- but for p/u exactly half way
+// between two integers, where it depends on R.  So a run of terms none of which
+// ties, that does not leave the power of two, changes R by the sum of the
+// rint(p/u), integers that add up exactly in any order.  Every wave adds up 1024
+// consecutive terms at acc's ulp; the waves' sums are taken in order, and a wave
+// whose terms tie or leave the power of two (or hold the hit) takes them in
+// chunks of 64 the same way, one term at a time where even that fails.  A sum
+// must end below 2^24 u, a remainder at 2^23 + 1 or above: then no value on the
+// way, before its rounding, was past the power of two.
+constexpr int kWalkU = 16, kWalkTerms = 64 * kWalkU;
+static_assert(kW == 16 && kWalkU == 16, "16 waves of 16 chunks: a row of 16 lanes holds one sum of each");
+enum WalkMode { kWalkSum, kWalkReach, kWalkDrain };
+
+struct WalkLds {
+    __attribute__((aligned(16))) float v[kWalkTerms];  // of the wave that walks its terms
+    float sum[kW], csum[kWalkU];                       // of the waves, of that wave's chunks
+    int tie[kW], ctie[kWalkU];
+    float acc;
+    int hit;
+};
+
+// u, 1/u for acc's ulp u; false where acc is negative, zero, tiny or not finite
+__device__ __forceinline__ bool ulp_of(float acc, float &u, float &inv) {
+    const uint32_t b = __float_as_uint(acc), e = b >> 23;
+    if (e < 25u || e >= 255u) return false;
+    u = __uint_as_float((e - 23u) << 23);
+    inv = __uint_as_float((277u - e) << 23);
+    return true;
+}
+
+// Takes the sums [next, n) of 16 runs of terms (lane l holds run l % 16's) into
+// R in order, as far as they need no closer look; returns the first not taken.
+template <WalkMode MODE>
+__device__ __forceinline__ int take_runs(float &R, float sum, bool tie, int next, int n, float u, float limit) {
+    const int l = threadIdx.x & 15;
+    const bool mine = l >= next;
+    float inc = mine ? sum : 0.0f;  // the sum of runs [next, l]
+    inc += dpp_f<0x111>(inc);       // row_shr 1, 2, 4, 8
+    inc += dpp_f<0x112>(inc);
+    inc += dpp_f<0x114>(inc);
+    inc += dpp_f<0x118>(inc);
+    const float R2 = MODE == kWalkDrain ? R - inc : R + inc;
+    bool ok = !tie && (MODE == kWalkDrain ? R2 >= 8388609.0f : R2 < 16777216.0f);
+    if (MODE == kWalkReach) ok = ok && R2 * u < limit;
+    const unsigned stop = (unsigned)__ballot(mine && !ok) & 0xffffu;
+    const int first = min(stop ? (int)__builtin_ctz(stop) : 16, n);
+    if (first > next) R = lane_value(R2, first - 1);
+    return first;
+}
+
+// the integers a lane's 4 consecutive terms change R by
+__device__ __forceinline__ float run_units(const f4 &v, float inv, bool &tie) {
+    float sum = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        const float t = v[c] * inv, r = rintf(t);
+        tie |= fabsf(t - r) == 0.5f;
+        sum += r;  // exact up to 2^24, not below it past that
+    }
+    return sum;
+}
+
+template <WalkMode MODE>
+__device__ __forceinline__ float walk(const float *__restrict__ p, int n, float acc, float limit, int *hit, WalkLds &s) {
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    *hit = -1;
+    f4 ahead[kWalkU / 4];
+    const auto fetch = [&](int base) {
+#pragma unroll
+        for (int j = 0; j < kWalkU / 4; j++) {
+            const int i = base + w * kWalkTerms + 256 * j + 4 * lane;
+            ahead[j] = *reinterpret_cast<const f4 *>(p + min(i, (n - 1) & ~3));
+        }
+    };
+    fetch(0);
+    for (int base = 0; base < n; base += kW * kWalkTerms) {
+        // terms that cannot change the sum any more
+        if (MODE != kWalkDrain && negligible(acc, p[base])) break;
+        const int wb = base + w * kWalkTerms, nw = min(kW, (n - base + kWalkTerms - 1) / kWalkTerms);
+        // the next round's terms are on their way while this one's are added
+        f4 v[kWalkU / 4];
+#pragma unroll
+        for (int j = 0; j < kWalkU / 4; j++) {
+            const int i = wb + 256 * j + 4 * lane;
+            v[j] = ahead[j];
+#pragma unroll
+            for (int c = 0; c < 4; c++) v[j][c] = i + c < n ? v[j][c] : 0.0f;  // adds nothing
+        }
+        fetch(base + kW * kWalkTerms);
+        int next = 0;  // the first wave whose terms are not in acc
+        while (next < nw) {
+            float u, inv;
+            if (ulp_of(acc, u, inv)) {
+                float sum = 0.0f;
+                bool tie = false;
+#pragma unroll
+                for (int j = 0; j < kWalkU / 4; j++) sum += run_units(v[j], inv, tie);
+                sum = wave_sum(sum);
+                const bool any = __any(tie);
+                if (lane == 0) {
+                    s.sum[w] = sum;
+                    s.tie[w] = any;
+                }
+                __syncthreads();
+                float R = acc * inv;
+                next = take_runs<MODE>(R, s.sum[lane & 15], s.tie[lane & 15] != 0, next, nw, u, limit);
+                acc = R * u;
+            }
+            if (next < nw && w == next) {
+                int h = -1;
+#pragma unroll
+                for (int j = 0; j < kWalkU / 4; j++) *reinterpret_cast<f4 *>(&s.v[256 * j + 4 * lane]) = v[j];
+                const int nc = min(kWalkU, (n - wb + 63) / 64);
+                for (int c = 0; c < nc && h < 0; c++) {
+                    float cu, cinv;
+                    if (ulp_of(acc, cu, cinv)) {
+                        // chunk 4j + lane / 16: a row of 16 lanes' float4 j
+#pragma unroll
+                        for (int j = 0; j < kWalkU / 4; j++) {
+                            bool tie = false;
+                            float sum = run_units(v[j], cinv, tie);
+                            sum += dpp_f<kDppQuadXor1>(sum);
+                            sum += dpp_f<kDppQuadXor2>(sum);
+                            sum += dpp_f<kDppRowHalfMirror>(sum);
+                            sum += dpp_f<kDppRowMirror>(sum);
+                            const unsigned ties = (unsigned)(__ballot(tie) >> (lane & 48)) & 0xffffu;
+                            if ((lane & 15) == 0) {
+                                s.csum[4 * j + (lane >> 4)] = sum;
+                                s.ctie[4 * j + (lane >> 4)] = ties != 0u;
+                            }
+                        }
+                        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                        __builtin_amdgcn_wave_barrier();
+                        float R = acc * cinv;
+                        c = take_runs<MODE>(R, s.csum[lane & 15], s.ctie[lane & 15] != 0, c, nc, cu, limit);
+                        acc = R * cu;
+                        if (c >= nc) break;
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    const float x = s.v[64 * c + lane];
+                    if (MODE == kWalkSum) {
+                        acc = chunk_end<false>(x, acc, 64);
+                    } else {
+                        const float run = chunk_record<MODE == kWalkDrain>(x, acc, 64);
+                        const unsigned long long at = __ballot((MODE == kWalkDrain ? run <= 0.0f : run >= limit) &&
+                                                               wb + 64 * c + lane < n);
+                        const int stop = at ? (int)__builtin_ctzll(at) : 63;
+                        if (at) h = wb + 64 * c + stop;
+                        acc = lane_value(run, stop);
+                    }
+                }
+                if (lane == 0) {
+                    s.acc = acc;
+                    s.hit = h;
+                }
+            }
+            __syncthreads();
+            if (next < nw) {
+                acc = s.acc;
+                if (s.hit >= 0) {
+                    *hit = s.hit;
+                    return acc;
+                }
+                next++;
+            }
+            __syncthreads();  // the next turn writes what was just read
+        }
+    }
+    return acc;
+}
+
+// The sum of the terms (src/sampler.rs:97) to walk[0], the first term to
+// walk[1].  NaN logits sort first or last (f32::total_cmp) and make an end term
+// NaN, as does an infinite maximum; then every probability is NaN.
+__global__ __launch_bounds__(kT) void sample_sum_kernel(SampleArgs a) {
+    __shared__ WalkLds s;
+    const int k = (int)top_k_of(a);
+    const float first = a.res_prob[0], last = a.res_prob[k - 1];
+    int hit;
+    const float sum = isnan(first) || isnan(last) ? first + last : walk<kWalkSum>(a.res_prob, k, -0.0f, 0.0f, &hit, s);
+    if (threadIdx.x == 0) {
+        a.walk[0] = sum;
+        a.walk[1] = first;
+    }
+}
+
+// The terms over their sum, and each workgroup's first position below min-p's
+// floor (src/sampler.rs:98-104).
+__global__ __launch_bounds__(kT) void sample_normalise_kernel(SampleArgs a) {
+    __shared__ int below;
+    const int k = (int)top_k_of(a), i = blockIdx.x * kT + threadIdx.x;
+    const float sum = a.walk[0], floor_p = a.walk[1] / sum * a.min_p;
+    if (threadIdx.x == 0) below = INT_MAX;
+    __syncthreads();
+    if (i < k) {
+        const float p = a.res_prob[i] / sum;
+        a.res_prob[i] = p;
+        if (a.min_p > 0.0f && p < floor_p) atomicMin(&below, i);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) a.tile_below[blockIdx.x] = below;
+}
+
+// top-p and the draw (src/sampler.rs:105-125).
+__global__ __launch_bounds__(kT) void sample_draw_kernel(SampleArgs a) {
+    __shared__ WalkLds s;
+    __shared__ int below;
+    const int k = (int)top_k_of(a);
+    if (threadIdx.x == 0) below = k;
+    uint64_t st[4] = {a.rng[0], a.rng[1], a.rng[2], a.rng[3]};
+    __syncthreads();
+    for (int b = threadIdx.x; b < (k + kT - 1) / kT; b += kT) atomicMin(&below, a.tile_below[b]);
+    __syncthreads();
+    int keep = max(below, 1), hit = -1;
+    const uint64_t u = next_u64(st);
+    if (!isnan(a.walk[0])) {
+        float total;
+        if (a.top_p < 1.0f) {
+            total = walk<kWalkReach>(a.res_prob, keep, 0.0f, a.top_p, &hit, s);
+            if (hit >= 0) keep = hit + 1;
+        } else {
+            total = walk<kWalkSum>(a.res_prob, keep, 0.0f, 0.0f, &hit, s);
+        }
+        const float r = (float)(uint32_t)(u >> 40) / 16777216.0f * total;
+        walk<kWalkDrain>(a.res_prob, keep, r, 0.0f, &hit, s);
+    }
+    const int pick = hit >= 0 ? hit : keep - 1;
+    __syncthreads();  // every thread has read the generator
+    if (threadIdx.x == 0) {
+        for (int j = 0; j < 4; j++) a.rng[j] = st[j];
+        *a.out = min(a.res_idx[pick], (uint32_t)a.vocab - 1u);
+        a.res_meta[0] = k;
+        a.res_meta[1] = keep;
+        a.res_meta[2] = 0;
+    }
+}
+
+hipError_t launch_sorted(const SampleArgs &a, hipStream_t s) {
+    const dim3 tiles((unsigned)((a.vocab + kTile - 1) / kTile)), block(kT);
+    hipLaunchKernelGGL(sort_hist_kernel<0>, tiles, block, 0, s, a);
+    hipLaunchKernelGGL(sort_move_kernel<0>, tiles, block, 0, s, a);
+    hipLaunchKernelGGL(sort_hist_kernel<1>, tiles, block, 0, s, a);
+    hipLaunchKernelGGL(sort_move_kernel<1>, tiles, block, 0, s, a);
+    hipLaunchKernelGGL(sort_hist_kernel<2>, tiles, block, 0, s, a);
+    hipLaunchKernelGGL(sort_move_kernel<2>, tiles, block, 0, s, a);
+    hipLaunchKernelGGL(sample_sum_kernel, dim3(1), block, 0, s, a);
+    hipLaunchKernelGGL(sample_normalise_kernel, dim3((top_k_of(a) + kT - 1) / kT), block, 0, s, a);
+    hipLaunchKernelGGL(sample_draw_kernel, dim3(1), block, 0, s, a);
+    return hipGetLastError();
+}
+
 }  // namespace
+
+// Draws that launch_sorted serves: more candidates than one workgroup selects
+// and sorts faster, which takes about 18 us + k/32 + vocab/10000 against 55-65
+// us + vocab/5000 (151936 ids: k 200 44 against 70 us, 1000 71 / 71, 2000 107 /
+// 76, all of them 2288 / 96; 20000 ids: k 1000 50 / 63, 2000 77 / 64; 5000 ids:
+// k 2000 53 / 58, 4000 92 / 59).  Up to kList ids every set fits its LDS.
+bool sorts_vocabulary(const SampleArgs &a) {
+    const uint32_t k = top_k_of(a);
+    return !(a.temperature <= 0.0f) && a.vocab > kList && k > (a.vocab > 16384 ? 1024u : 2048u);
+}
 
 hipError_t launch_sample(const SampleArgs &a, hipStream_t s) {
     // the split kernel is needed for the penalty, greedy, and the split top-k
@@ -737,6 +1187,7 @@ hipError_t launch_sample(const SampleArgs &a, hipStream_t s) {
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
+    if (sorts_vocabulary(a)) return launch_sorted(a, s);
     hipLaunchKernelGGL(sample_kernel, dim3(1), dim3(kT), 0, s, a);
     return hipGetLastError();
 }

@@ -27,6 +27,7 @@ struct wick_hip_sampler {
     uint32_t *part_id = nullptr;
     unsigned long long *part_cand = nullptr;
     int *part_count = nullptr;
+    uint32_t *tiles = nullptr;  // SampleArgs' tile_hist, tile_least, tile_below and walk
     // staging for the host-array entry point
     float *logits = nullptr;
     uint32_t *out = nullptr;
@@ -62,7 +63,8 @@ void seed_rng(uint64_t seed, uint64_t out[4]) {
 
 void release(wick_hip_sampler *s) {
     void *bufs[] = {s->flags, s->rng,      s->key0,     s->key1,      s->idx1,       s->res_idx, s->res_prob, s->meta,
-                    s->part_val, s->part_id, s->part_cand, s->part_count, s->logits, s->out,     s->history};
+                    s->part_val, s->part_id, s->part_cand, s->part_count, s->tiles,
+                    s->logits,   s->out,     s->history};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
 }
@@ -109,6 +111,11 @@ int sampler_enqueue(wick_hip_sampler *s, float *logits, const uint32_t *history,
     a.part_id = s->part_id;
     a.part_cand = s->part_cand;
     a.part_count = s->part_count;
+    const size_t tiles = ((size_t)s->vocab + kSampleTile - 1) / kSampleTile;
+    a.tile_hist = reinterpret_cast<uint16_t *>(s->tiles);
+    a.tile_least = s->tiles + tiles * 1024;
+    a.tile_below = reinterpret_cast<int *>(a.tile_least + tiles);
+    a.walk = reinterpret_cast<float *>(a.tile_below + tiles * (kSampleTile / 1024));
     hipError_t e = launch_sample(a, s->stream);
     if (e != hipSuccess) return hip_fail(e, "sample launch");
     return WICK_HIP_OK;
@@ -138,15 +145,17 @@ int wick_hip_sampler_create(const wick_hip_sampler_config *cfg, int vocab, void 
     s->slice = ((vocab + s->parts - 1) / s->parts + 31) / 32 * 32;
     s->parts = (vocab + s->slice - 1) / s->slice;
     const size_t n = (size_t)vocab, words = (n + 31) / 32, np = wick::kSampleParts;
+    const size_t tiles = (n + wick::kSampleTile - 1) / wick::kSampleTile;
     struct {
         void **p;
         size_t bytes;
-    } want[] = {{(void **)&s->flags, words * 4},   {(void **)&s->rng, 32},        {(void **)&s->key0, n * 4},
-                {(void **)&s->key1, n * 4},        {(void **)&s->idx1, n * 4},    {(void **)&s->res_idx, n * 4},
-                {(void **)&s->res_prob, n * 4},    {(void **)&s->meta, 16},       {(void **)&s->logits, n * 4},
+    } want[] = {{(void **)&s->flags, words * 4},   {(void **)&s->rng, 32},        {(void **)&s->key0, n * 8},
+                {(void **)&s->key1, n * 8},        {(void **)&s->idx1, n * 4},    {(void **)&s->res_idx, n * 4},
+                {(void **)&s->res_prob, (n + 3) / 4 * 16},    {(void **)&s->meta, 16},       {(void **)&s->logits, n * 4},
                 {(void **)&s->out, 16},            {(void **)&s->part_val, np * 4},
                 {(void **)&s->part_id, np * 4},    {(void **)&s->part_cand, np * wick::kFastK * 8},
-                {(void **)&s->part_count, np * 4}};
+                {(void **)&s->part_count, np * 4},
+                {(void **)&s->tiles, (tiles * (1024 + 1 + wick::kSampleTile / 1024) + 4) * 4}};
     int rc = WICK_HIP_OK;
     for (auto &w : want) {
         hipError_t e = hipMalloc(w.p, w.bytes);

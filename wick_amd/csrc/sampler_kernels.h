@@ -10,6 +10,7 @@ namespace wick {
 
 constexpr int kSampleParts = 16;  // most workgroups of the split kernel
 constexpr int kFastK = 64;        // top-k up to this is taken per slice, then merged
+constexpr int kSampleTile = 4096;  // ids per workgroup of the whole-vocabulary sort
 constexpr int kSliceMax = 12288;  // longest slice whose keys the split kernel holds in registers
 
 // One draw of Sampler::sample (/root/reference/src/sampler.rs:73-127).
@@ -24,10 +25,11 @@ struct SampleArgs {
     float temperature, top_p, min_p, penalty;
     uint32_t top_k;
     // Candidate sets larger than the in-LDS list are radix-sorted in global
-    // memory: keys in key0/key1, ids in res_idx/idx1 ([vocab] each).
+    // memory: keys in key0/key1, ids in res_idx/idx1 ([vocab] each), or pairs of
+    // both in key0/key1 ([2 * vocab]) in the sort over many workgroups.
     uint32_t *key0, *key1, *idx1;
     uint32_t *res_idx;  // [vocab] the candidates in wick's order
-    float *res_prob;    // [vocab] their probabilities after normalisation
+    float *res_prob;    // [vocab], readable to a multiple of 4: their probabilities after normalisation
     int *res_meta;      // {k, keep, internal check (0 = ok)}
     // The split kernel: `parts` slices of `slice` ids (a multiple of 32), each
     // leaving its argmax in part_val/part_id or its k best (key << 32 | id) in
@@ -39,6 +41,13 @@ struct SampleArgs {
     uint32_t *part_id;
     unsigned long long *part_cand;
     int *part_count;
+    // The sort of the whole vocabulary, per tile of kSampleTile ids: up to 2^11
+    // digit counts, the least key, the first position below min-p's floor (one per
+    // 1024 candidates); walk: the sum of the terms, the first term.
+    uint16_t *tile_hist;
+    uint32_t *tile_least;
+    int *tile_below;
+    float *walk;
 };
 
 hipError_t launch_sample(const SampleArgs &a, hipStream_t s);
