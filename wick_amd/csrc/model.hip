@@ -337,12 +337,14 @@ __global__ __launch_bounds__(256) void gemv1_kernel(const GemvArgs a) {
 // length from L2.  In the MFMA lane layout consecutive lanes are consecutive
 // rows, and the L1 then serves one lane (16 bytes) a cycle: 64 cache accesses
 // per load instruction counted, 13.5 bytes per cycle and CU whatever the tile.
-// So a wave loads each 16 x 16 block with 4 consecutive lanes on one row's 64
-// bytes (16 accesses) and passes it through its own piece of LDS.  256 tokens
-// of a 2048-wide layer (hidden 2048, FFN 5632): q/k/v 60 -> 27.6 us, o 22.5,
-// gate/up 194 -> 108, down 57 (o and down together 180 -> 80); without the
-// LDS turn 31, 27, 115, 69.  251 tokens at hidden 576, FFN 1536: 10.8 -> 5.8,
-// 6.2, 21.6 -> 14.7, 10.0 us.
+// So a wave loads 16 rows x 32 k with 8 consecutive lanes on one row's 128-byte
+// line (4 lanes on 64 bytes: 5 to 20% slower) and passes it through its own
+// piece of LDS.  251 tokens of a 2048-wide layer (hidden 2048, FFN 5632): q/k/v
+// 60 -> 27.5 us, o and down 180 together -> 20.7 + 47.3 (122 TFLOP/s; the
+// library's largest f32 products reach 152), gate/up 194 -> 110; straight to
+// registers 31, 27 + 69, 115.  251 tokens at hidden 576, FFN 1536: 10.8 -> 5.8,
+// 6.3, 21.6 -> 14.1, 9.5 us.  Reading the next fragments from LDS ahead of the
+// products gained nothing.
 __device__ __forceinline__ f4 mfma4(float a, float b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t gemm_rsrc(const float *base, unsigned bytes) {
@@ -395,8 +397,10 @@ __global__ __launch_bounds__(64 * NW) void gemm_kernel(const GemvArgs a) {
     for (int r = 0; r < RB; r++) so_w[r] = __builtin_amdgcn_readfirstlane(16 * r < wrows ? 16u * r * pitch : 0u);
 #pragma unroll
     for (int t = 0; t < TB; t++) so_x[t] = __builtin_amdgcn_readfirstlane(16 * t < toks ? 16u * t * pitch : 0u);
-    // the row and 16-byte chunk this lane loads of each 16 x 16 block
-    const int lr = lane >> 2, lc = (lane & 3) ^ ((lr >> 1) & 3);
+    // the row (of the first 8, or of the last 8) and 16-byte chunk this lane
+    // loads of 16 rows x 32 k
+    static_assert(KU % 2 == 0, "batches of whole cache lines");
+    const int lr = lane >> 3, lc = (lane & 7) ^ lr;  // (row & 7 is lr in both halves)
     const unsigned vrow = (unsigned)lr * pitch + 16u * lc;
 
     struct Batch {
@@ -405,8 +409,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_kernel(const GemvArgs a) {
     auto load = [&](Batch &b, int n) {
 #pragma unroll
         for (int u = 0; u < KU; u++) {
-            const int k = 16 * (KU * n + u);
-            const unsigned vo = k + 4 * lc < a.cols ? vrow + 4u * (unsigned)k : 0x80000000u;
+            const int k = 16 * (KU * n + (u & ~1));
+            const unsigned vo = (k + 4 * lc < a.cols ? vrow + 4u * (unsigned)k : 0x80000000u) + (u & 1) * 8u * pitch;
 #pragma unroll
             for (int r = 0; r < RB; r++) {
                 b.w[0][u][r] = gemm_load(rw, vo, so_w[r]);
@@ -420,19 +424,19 @@ __global__ __launch_bounds__(64 * NW) void gemm_kernel(const GemvArgs a) {
     // through the wave's own LDS: stored as loaded, read in the product's lane
     // layout (one wave's LDS operations run in order, so no barrier)
     f4 *const mine = &sm[w][0];
-    const int rd = 4 * i + (g ^ ((i >> 1) & 3));
+    const int rd[2] = {8 * i + (g ^ (i & 7)), 8 * i + ((4 + g) ^ (i & 7))};
     auto turn = [&](Batch &b) {
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int u = 0; u < KU; u++) {
-            f4 *q = mine + 64 * u * (M * RB + TB);
+            f4 *q = mine + 64 * ((u & ~1) * (M * RB + TB) + (u & 1));
 #pragma unroll
             for (int m = 0; m < M; m++)
 #pragma unroll
-                for (int r = 0; r < RB; r++) q[64 * (m * RB + r) + lane] = b.w[m][u][r];
+                for (int r = 0; r < RB; r++) q[128 * (m * RB + r) + lane] = b.w[m][u][r];
 #pragma unroll
-            for (int t = 0; t < TB; t++) q[64 * (M * RB + t) + lane] = b.x[u][t];
+            for (int t = 0; t < TB; t++) q[128 * (M * RB + t) + lane] = b.x[u][t];
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -440,13 +444,13 @@ __global__ __launch_bounds__(64 * NW) void gemm_kernel(const GemvArgs a) {
     auto frags = [&](Batch &b) {
 #pragma unroll
         for (int u = 0; u < KU; u++) {
-            const f4 *q = mine + 64 * u * (M * RB + TB) + rd;
+            const f4 *q = mine + 64 * (u & ~1) * (M * RB + TB) + rd[u & 1];
 #pragma unroll
             for (int m = 0; m < M; m++)
 #pragma unroll
-                for (int r = 0; r < RB; r++) b.w[m][u][r] = q[64 * (m * RB + r)];
+                for (int r = 0; r < RB; r++) b.w[m][u][r] = q[128 * (m * RB + r)];
 #pragma unroll
-            for (int t = 0; t < TB; t++) b.x[u][t] = q[64 * (M * RB + t)];
+            for (int t = 0; t < TB; t++) b.x[u][t] = q[128 * (M * RB + t)];
         }
     };
     f4 acc[M][RB][TB];
@@ -807,46 +811,59 @@ hipError_t launch_gemv(int epi, const GemvArgs &a, hipStream_t s) {
 
 namespace {
 
-template <int EPI, int RB, int TB, int KU>
+template <int EPI, int RB, int TB, int NW, int KU>
 hipError_t gemm_launch(const GemvArgs &a, hipStream_t s) {
-    constexpr int NW = 8;
     const int nrt = (a.rows + 16 * RB - 1) / (16 * RB), ntt = (a.t + 16 * TB - 1) / (16 * TB);
     hipLaunchKernelGGL((gemm_kernel<EPI, RB, TB, NW, KU>), dim3(8u * ((nrt + 7) / 8) * ntt), dim3(64 * NW), 0, s, a);
     return hipGetLastError();
 }
 
-// What a tile of rb x tb blocks (of m weight matrices) costs: the products of
-// the busiest of the 256 CUs, each dearer the less the tile reuses what it
-// loads.  The model's order is the measured one where the tiles differ by more
-// than a few percent: 64 tokens at 2048 x 2048: 1x2 11.7 us, 2x2 15; 251
-// tokens at 2560 x 2048: 5x2 27.6, 2x2 32.4, 1x2 33+; at 2048 x 5632: 2x4 52.7,
-// 2x2 57; at 576 x 576: 1x2 and 2x2 6.2, 2x4 8.  (Gate/up on 2x4 blocks of both
-// matrices fills a CU's LDS with one workgroup: 113 us against 108 on 2x2.)
-double gemm_cost(const GemvArgs &a, int m, int rb, int tb) {
+// 8 waves, or 6 where those take no more batches of 32 columns each (576 columns
+// are 18: 3 either way; 16 tokens of gate/up 6.2 against 6.5 us, 251 tokens of o
+// 6.3 against 6.5; where they take more, up to a quarter slower).
+template <int EPI, int RB, int TB>
+hipError_t gemm_waves(const GemvArgs &a, hipStream_t s) {
+    const int nbat = (a.cols + 31) / 32;
+    if ((nbat + 5) / 6 == (nbat + 7) / 8) return gemm_launch<EPI, RB, TB, 6, 2>(a, s);
+    return gemm_launch<EPI, RB, TB, 8, 2>(a, s);
+}
+
+// What a tile of rb x tb blocks costs: the products of the busiest of the 256
+// CUs, each dearer the less the tile reuses what it loads.  The model's order
+// is the measured one where the tiles differ by more than a few percent: 64
+// tokens at 2048 x 2048: 1x2 10 us, 2x2 12.6; 251 tokens at 2560 x 2048: 5x2
+// 27.5, 1x2 30.2, 2x2 30.7; at 2048 x 5632: 2x4 47.3, 2x2 50.4; at 576 x 576:
+// 2x2 6.3, 1x2 6.6, 2x4 8.
+double gemm_cost(const GemvArgs &a, int rb, int tb) {
     const long long wgs = (long long)((a.rows + 16 * rb - 1) / (16 * rb)) * ((a.t + 16 * tb - 1) / (16 * tb));
-    return (double)((wgs + 255) / 256) * (m * rb * tb + 0.5 * (m * rb + tb));
+    return (double)((wgs + 255) / 256) * (rb * tb + 0.5 * (rb + tb));
 }
 
 template <int EPI>
 hipError_t gemm_epi(const GemvArgs &a, hipStream_t s) {
-    constexpr int m = EPI == kEpiSwiglu ? 2 : 1;
     if (a.t <= 16) {
         // bound by the weights' arrival: more of them in flight per wave where a
-        // wave takes several batches (4 tokens, 2048 x 5632: 13.9 against 17.6
-        // us; at 576 columns a batch of 4 leaves waves idle, 4.3 against 3.6)
-        if constexpr (m == 1)
-            if (a.cols >= 2048) return gemm_launch<EPI, 1, 1, 4>(a, s);
-        return gemm_launch<EPI, 1, 1, 2>(a, s);
+        // wave takes several batches (4 tokens, 2048 x 5632: 13.7 against 17.4
+        // us; at 576 columns a batch of 4 leaves waves idle, 4.1 against 3.5)
+        if constexpr (EPI != kEpiSwiglu)
+            if (a.cols >= 2048) return gemm_launch<EPI, 1, 1, 8, 4>(a, s);
+        return gemm_waves<EPI, 1, 1>(a, s);
     }
-    const int tiles[][2] = {{1, 2}, {2, 2}, {2, 4}, {5, 2}};
-    int best = 0;
-    for (int i = 1; i < (m == 2 ? 2 : 4); i++)
-        if (gemm_cost(a, m, tiles[i][0], tiles[i][1]) < gemm_cost(a, m, tiles[best][0], tiles[best][1])) best = i;
-    if constexpr (m == 1) {
-        if (best == 3) return gemm_launch<EPI, 5, 2, 1>(a, s);
-        if (best == 2) return gemm_launch<EPI, 2, 4, 1>(a, s);
+    if constexpr (EPI == kEpiSwiglu) {
+        // Larger tiles of both matrices fill a CU's LDS with one workgroup: 251
+        // tokens at 5632 x 2048 114 us on 2x2 against 110.  8 waves leave room
+        // for two, worth it where a wave takes many batches (at 1536 x 576 21
+        // against 14.1 us on 4 waves; at 5632 x 2048 110 against 118).
+        return a.cols < 1024 ? gemm_launch<EPI, 1, 2, 4, 2>(a, s) : gemm_launch<EPI, 1, 2, 8, 2>(a, s);
+    } else {
+        const int tiles[][2] = {{1, 2}, {2, 2}, {2, 4}, {5, 2}};
+        int best = 0;
+        for (int i = 1; i < 4; i++)
+            if (gemm_cost(a, tiles[i][0], tiles[i][1]) < gemm_cost(a, tiles[best][0], tiles[best][1])) best = i;
+        if (best == 3) return gemm_launch<EPI, 5, 2, 8, 2>(a, s);
+        if (best == 2) return gemm_launch<EPI, 2, 4, 8, 2>(a, s);
+        return best == 1 ? gemm_waves<EPI, 2, 2>(a, s) : gemm_waves<EPI, 1, 2>(a, s);
     }
-    return best == 1 ? gemm_launch<EPI, 2, 2, 1>(a, s) : gemm_launch<EPI, 1, 2, 1>(a, s);
 }
 
 }  // namespace
