@@ -506,3 +506,31 @@ def test_products_of_several_tokens(hidden, ff, vocab, t):
         again = m.forward(m.new_cache(t), toks[3:], all_logits=True)
     assert np.abs(got - want).max() < 1e-4
     assert np.abs(again - alone).max() < 1e-4
+
+
+@pytest.mark.parametrize("heads,kvh,n", [(9, 3, 100), (14, 2, 260), (3, 1, 500), (16, 2, 1000), (36, 2, 130)])
+def test_o_product_merges_the_chunks(heads, kvh, n):
+    """Single-token steps over 2 to 17 chunks of 64 positions, whose states the o product
+    merges up to 16 (and up to 1024 columns: not the last shape's 2304): each step's logits
+    within 1e-4 of the CPU oracle and the same greedy ids through decode()'s replayed steps,
+    across the lengths where the number of chunks changes."""
+    cfg = Config("llama", 128, 96, 2, heads, kvh, 64, 300, rms_eps=1e-5, rope_theta=10000.0)
+    w = random_weights(cfg, seed=heads + n, std=0.05)
+    prompt = [int(x) for x in random_prompt(n, n, cfg.vocab)]
+    om = ol.OracleModel(cfg, w)
+    ost = om.new_state(n + 64)
+    want = om.forward(ost, prompt)
+    ids = []
+    with DeviceModel(cfg, w) as m:
+        cache = m.new_cache(n + 64)
+        cache.set_option(_native.OPT_DECODE_CHUNK, 64)
+        got = m.forward(cache, prompt)
+        for step in range(60):
+            diff = np.abs(got[0] - want[0]).max()
+            assert diff < 1e-4, f"step {step}: logits differ by {diff}"
+            ids.append(ol.argmax(want[0]))
+            got = m.forward(cache, [ids[-1]])
+            want = om.forward(ost, [ids[-1]])
+        cache.len = 0
+        first = m.prefill(cache, prompt)
+        assert [first] + m.decode(cache, first, 59) == ids

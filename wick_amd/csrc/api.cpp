@@ -353,6 +353,7 @@ int run_prep(wick_hip_kv *kv, int layer, int heads, float *q_dev, const float *k
 
 // One token: the preparation fused into the decode kernel's prologue (q from
 // the raw projections, k and v appended at position start), then attention.
+// att_dev == nullptr: the states of several chunks stay unmerged in the workspace.
 int run_decode_fused(wick_hip_kv *kv, int layer, int heads, const float *q_raw, const float *k_raw,
                      const float *v_raw, int start, float *att_dev, const int *len_dev) {
     PrepConsts c;
@@ -450,6 +451,32 @@ int attend_model_oproj(wick_hip_kv *kv, int layer, int heads, float *q_dev, cons
     hipError_t e = wick::launch_decode_oproj(kv->head_dim, a, kv->stream);
     if (e != hipSuccess) return hip_fail(e, "decode + output projection launch");
     *units_out = kv->kv_heads * hslices;
+    return WICK_HIP_OK;
+}
+
+int attend_model_states(wick_hip_kv *kv, int layer, int heads, float *q_dev, const float *k_dev, const float *v_dev,
+                        int start, DecodeStates *out, const int *len_dev) {
+    int rc = check_kv(kv, layer);
+    if (rc) return rc;
+    if ((rc = check_span(kv, start, 1))) return rc;
+    if (!q_dev || !k_dev || !v_dev || !out) return fail(WICK_HIP_EINVAL, "null argument");
+    if ((rc = check_aligned(q_dev, "q_dev")) || (rc = check_aligned(k_dev, "k_dev")) ||
+        (rc = check_aligned(v_dev, "v_dev")))
+        return rc;
+    if (heads < 1 || heads % kv->kv_heads != 0)
+        return fail(WICK_HIP_EINVAL, "heads (%d) must be a positive multiple of kv_heads (%d)", heads, kv->kv_heads);
+    const int group = heads / kv->kv_heads;
+    const int hslices = (group + wick::kTileRows - 1) / wick::kTileRows, units = kv->kv_heads * hslices;
+    int chunk, nchunks;
+    plan_chunks(kv, units, start + 1, &chunk, &nchunks);
+    if (kv->head_dim != 64 || nchunks < 2 || nchunks > wick::kStateChunks || heads * kv->head_dim > wick::kStateCols)
+        return 1;
+    if ((rc = run_decode_fused(kv, layer, heads, q_dev, k_dev, v_dev, start, nullptr, len_dev))) return rc;
+    wick::decode_workspace_parts(kv->part, units, kv->head_dim, out);
+    out->head_dim = kv->head_dim;
+    out->group = group;
+    out->hslices = hslices;
+    out->nchunks = nchunks;
     return WICK_HIP_OK;
 }
 

@@ -828,6 +828,13 @@ size_t decode_workspace_floats(int units, int head_dim) {
     return (size_t)units * 16 * kDecodeMaxChunks * (head_dim + 2);
 }
 
+void decode_workspace_parts(const float *part, int units, int head_dim, DecodeStates *out) {
+    out->o = part;
+    out->m = part + (size_t)units * 16 * kDecodeMaxChunks * head_dim;
+    out->l = out->m + (size_t)units * 16 * kDecodeMaxChunks;
+    out->stride = kDecodeMaxChunks;
+}
+
 template <int D>
 struct DecodeSpace {
     float *o, *m, *l;
@@ -1772,7 +1779,7 @@ hipError_t launch_decode(int head_dim, const DecodeArgs &a, int grid, hipStream_
     default: return hipErrorInvalidValue;
     }
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess || a.nchunks == 1) return e;
+    if (e != hipSuccess || a.nchunks == 1 || !a.att) return e;
     const dim3 mgrid((unsigned)(a.kv_heads * a.group * (head_dim / 16)));
     // 16 thread groups x NB child slots cover the chunks
     const int nb = a.nchunks <= 16 ? 1 : a.nchunks <= 32 ? 2 : a.nchunks <= 64 ? 4 : a.nchunks <= 128 ? 8 : 16;

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 
+#include "model_kernels.h"
 #include "wick_hip.h"
 
 namespace wick {
@@ -122,8 +123,11 @@ int prefill_blocks_per_cu(int head_dim, int rows32);
 // Whether the prefill kernel for this shape can take two row blocks per workgroup.
 bool prefill_has_rows32(int head_dim, int capacity);
 
-// Launches decode_kernel and, when it splits the keys, decode_merge_kernel.
+// Launches decode_kernel and, when it splits the keys and a.att is not null,
+// decode_merge_kernel.
 hipError_t launch_decode(int head_dim, const DecodeArgs &a, int grid, hipStream_t s);
+// The workspace's three parts (DecodeStates' o, m, l) for `units`.
+void decode_workspace_parts(const float *part, int units, int head_dim, DecodeStates *out);
 // Whether decode_kernel's fused output projection serves this plan (head_dim
 // 64 or 128, one chunk of at most kOprojMaxChunk keys per unit, the unit's
 // columns fit kOprojChunks).
@@ -167,6 +171,13 @@ int attend_model(wick_hip_kv *kv, int layer, int heads, float *q_dev, const floa
 int attend_model_oproj(wick_hip_kv *kv, int layer, int heads, float *q_dev, const float *k_dev, const float *v_dev,
                        int start, const float *wo, int hidden, float *oparts, int *units_out,
                        const int *len_dev = nullptr);
+
+// attend_model for one token without the merge of its chunks' states, at
+// head_dim 64 where there are 2 to kStateChunks of them and at most kStateCols
+// columns: *out describes the states, valid until the next call on the cache.  Returns
+// WICK_HIP_OK, or 1 (nothing launched) when the shape is another.
+int attend_model_states(wick_hip_kv *kv, int layer, int heads, float *q_dev, const float *k_dev, const float *v_dev,
+                        int start, DecodeStates *out, const int *len_dev = nullptr);
 
 // The decode launch plan (chunk size and count) for `heads` query heads over
 // len cached positions: equal keys launch the same kernels on the same grids.

@@ -320,6 +320,65 @@ __global__ __launch_bounds__(256) void gemv1_kernel(const GemvArgs a) {
     }
 }
 
+// The o product of a split single-token decode with the merge of its chunks'
+// states (DecodeStates) as the prologue: gemv1_kernel<1, UNR, kEpiResid> whose
+// input row every workgroup merges for itself.  Thread t owns float4s t, t + 256,
+// ... of the row: it requests all NC states of its float4 (slots past nchunks
+// repeat the last and weigh 0) next to the weights, so the kernel waits for
+// memory once (figures at kStateChunks).
+template <int UNR, int NC>
+__global__ __launch_bounds__(256) void gemv1_states_kernel(const GemvArgs a, const DecodeStates st) {
+    constexpr int XK = (64 * UNR + 255) / 256;
+    __shared__ f4 sx[256 * XK];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, t = threadIdx.x;
+    const int row = blockIdx.x * 4 + w;
+    const int C4 = a.cols >> 2;
+    const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    f4 wv[UNR];
+    const f4 *W = reinterpret_cast<const f4 *>(a.w + (size_t)min(row, a.rows - 1) * a.cols);
+#pragma unroll
+    for (int u = 0; u < UNR; u++) wv[u] = __builtin_nontemporal_load(W + min(lane + 64 * u, C4 - 1));
+    const float resid = (a.resid ? a.resid : a.out0)[min(row, a.rows - 1)];
+#pragma unroll
+    for (int k = 0; k < XK; k++) {
+        const int c = min(t + 256 * k, C4 - 1), h = 4 * c / st.head_dim, d = 4 * c % st.head_dim;
+        const int kvh = h / st.group, hh = h % st.group;
+        const size_t base = (size_t)((kvh * st.hslices + hh / 16) * 16 + hh % 16) * st.stride;
+        f4 o[NC];
+        float m[NC], l[NC];
+#pragma unroll
+        for (int j = 0; j < NC; j++) {
+            const size_t at = base + min(j, st.nchunks - 1);
+            m[j] = st.m[at];
+            l[j] = st.l[at];
+            o[j] = *reinterpret_cast<const f4 *>(st.o + at * st.head_dim + d);
+        }
+        float M = m[0];
+#pragma unroll
+        for (int j = 1; j < NC; j++) M = fmaxf(M, m[j]);
+        f4 acc = zero;
+        float L = 0.0f;
+#pragma unroll
+        for (int j = 0; j < NC; j++) {
+            const float e = j < st.nchunks ? __builtin_amdgcn_exp2f(m[j] - M) : 0.0f;
+            acc += o[j] * e;
+            L += l[j] * e;
+        }
+        sx[t + 256 * k] = acc / L;
+    }
+    __syncthreads();
+    if (row >= a.rows) return;
+    float acc = 0.0f;
+#pragma unroll
+    for (int u = 0; u < UNR; u++) {
+        const int c = lane + 64 * u;
+        if (c >= C4) break;
+        acc = dot4(wv[u], sx[c], acc);
+    }
+    acc = wave_sum(acc);
+    if (lane == 0) a.out0[row] = resid + acc;
+}
+
 // Several tokens: out rows of W . X^T on the f32 matrix cores
 // (v_mfma_f32_16x16x4_f32: A = 16 weight rows x 4 k, B = 4 k x 16 tokens).  The
 // contraction index is permuted so each lane loads whole float4s: MFMA e of
@@ -362,7 +421,7 @@ __device__ __forceinline__ f4 gemm_load(__amdgpu_buffer_rsrc_t r, unsigned voff,
 }
 
 template <int EPI, int RB, int TB, int NW, int KU>
-__global__ __launch_bounds__(64 * NW) void gemm_kernel(const GemvArgs a) {
+__global__ __launch_bounds__(64 * NW) void gemm_kernel(const GemmArgs a) {
     constexpr int M = EPI == kEpiSwiglu ? 2 : 1;  // weight matrices
     constexpr int NB = RB * TB;                   // 16 x 16 blocks of the tile
     constexpr int NT = 16 * TB;                   // tokens of the tile
@@ -580,7 +639,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_kernel(const GemvArgs a) {
 
 // step (graph-replayed decode loop): the token is tokens[*step + i].
 // xg: also x * xnorm (the first layer's norm weight) and the row's sum of
-// squares, for the products that apply the norm's factor (GemvArgs::ssq).
+// squares, for the products that apply the norm's factor (GemmArgs::ssq).
 __global__ __launch_bounds__(256) void embed_kernel(const float *__restrict__ embed, const uint32_t *__restrict__ tokens,
                                                     const int *__restrict__ step, float *__restrict__ x, int hidden,
                                                     float *__restrict__ xg, const float *__restrict__ xnorm,
@@ -790,6 +849,29 @@ hipError_t gemv_epi(const GemvArgs &a, hipStream_t s) {
 
 }  // namespace
 
+template <int UNR>
+static hipError_t gemv1_states_launch(const GemvArgs &a, const DecodeStates &st, hipStream_t s) {
+    const dim3 grid((unsigned)((a.rows + 3) / 4)), block(256);
+    if (st.nchunks <= 4)
+        hipLaunchKernelGGL((gemv1_states_kernel<UNR, 4>), grid, block, 0, s, a, st);
+    else if (st.nchunks <= 8)
+        hipLaunchKernelGGL((gemv1_states_kernel<UNR, 8>), grid, block, 0, s, a, st);
+    else
+        hipLaunchKernelGGL((gemv1_states_kernel<UNR, kStateChunks>), grid, block, 0, s, a, st);
+    return hipGetLastError();
+}
+
+hipError_t launch_gemv_states(const GemvArgs &a, const DecodeStates &st, hipStream_t s) {
+    if (a.rows <= 0) return hipSuccess;
+    if (a.t != 1 || a.norm || a.cols > kStateCols || st.nchunks < 1 || st.nchunks > kStateChunks)
+        return hipErrorInvalidValue;
+    // the fewest spare slots of a row's float4s (gemv1_launch)
+    const int need = ((a.cols >> 2) + 63) / 64;
+    if (need <= 2) return gemv1_states_launch<2>(a, st, s);
+    if (need <= 3) return gemv1_states_launch<3>(a, st, s);
+    return gemv1_states_launch<4>(a, st, s);
+}
+
 hipError_t launch_gemv(int epi, const GemvArgs &a, hipStream_t s) {
     if (a.rows <= 0 || a.t <= 0) return hipSuccess;
     if (a.parts) {
@@ -812,7 +894,7 @@ hipError_t launch_gemv(int epi, const GemvArgs &a, hipStream_t s) {
 namespace {
 
 template <int EPI, int RB, int TB, int NW, int KU>
-hipError_t gemm_launch(const GemvArgs &a, hipStream_t s) {
+hipError_t gemm_launch(const GemmArgs &a, hipStream_t s) {
     const int nrt = (a.rows + 16 * RB - 1) / (16 * RB), ntt = (a.t + 16 * TB - 1) / (16 * TB);
     hipLaunchKernelGGL((gemm_kernel<EPI, RB, TB, NW, KU>), dim3(8u * ((nrt + 7) / 8) * ntt), dim3(64 * NW), 0, s, a);
     return hipGetLastError();
@@ -822,7 +904,7 @@ hipError_t gemm_launch(const GemvArgs &a, hipStream_t s) {
 // are 18: 3 either way; 16 tokens of gate/up 6.2 against 6.5 us, 251 tokens of o
 // 6.3 against 6.5; where they take more, up to a quarter slower).
 template <int EPI, int RB, int TB>
-hipError_t gemm_waves(const GemvArgs &a, hipStream_t s) {
+hipError_t gemm_waves(const GemmArgs &a, hipStream_t s) {
     const int nbat = (a.cols + 31) / 32;
     if ((nbat + 5) / 6 == (nbat + 7) / 8) return gemm_launch<EPI, RB, TB, 6, 2>(a, s);
     return gemm_launch<EPI, RB, TB, 8, 2>(a, s);
@@ -834,13 +916,13 @@ hipError_t gemm_waves(const GemvArgs &a, hipStream_t s) {
 // tokens at 2048 x 2048: 1x2 10 us, 2x2 12.6; 251 tokens at 2560 x 2048: 5x2
 // 27.5, 1x2 30.2, 2x2 30.7; at 2048 x 5632: 2x4 47.3, 2x2 50.4; at 576 x 576:
 // 2x2 6.3, 1x2 6.6, 2x4 8.
-double gemm_cost(const GemvArgs &a, int rb, int tb) {
+double gemm_cost(const GemmArgs &a, int rb, int tb) {
     const long long wgs = (long long)((a.rows + 16 * rb - 1) / (16 * rb)) * ((a.t + 16 * tb - 1) / (16 * tb));
     return (double)((wgs + 255) / 256) * (rb * tb + 0.5 * (rb + tb));
 }
 
 template <int EPI>
-hipError_t gemm_epi(const GemvArgs &a, hipStream_t s) {
+hipError_t gemm_epi(const GemmArgs &a, hipStream_t s) {
     if (a.t <= 16) {
         // bound by the weights' arrival: more of them in flight per wave where a
         // wave takes several batches (4 tokens, 2048 x 5632: 13.7 against 17.4
@@ -868,7 +950,7 @@ hipError_t gemm_epi(const GemvArgs &a, hipStream_t s) {
 
 }  // namespace
 
-hipError_t launch_gemm(int epi, const GemvArgs &a, hipStream_t s) {
+hipError_t launch_gemm(int epi, const GemmArgs &a, hipStream_t s) {
     if (a.rows <= 0 || a.t <= 0) return hipSuccess;
     // 80 rows of a tile within a signed 32-bit byte range
     if (a.cols % 4 != 0 || a.cols > (1 << 22) || a.norm) return hipErrorInvalidValue;

@@ -12,7 +12,8 @@
 // For one token over a short cache (one decode chunk per unit, head_dim 64 or
 // 128, small GQA groups) the attention and the wo product are one launch that
 // writes each unit's partial product, and the gate/up product adds those to
-// the residual as its prologue: four launches per layer instead of five.
+// the residual as its prologue: four launches per layer instead of five.  Over
+// a few chunks the wo product merges their states: five instead of six.
 // then the final norm + LM head (:507-515) and, for the greedy entry points,
 // sampler::argmax (src/sampler.rs:129-137), all on the model's stream.
 #include "wick_hip_model.h"
@@ -183,13 +184,13 @@ int check_cache(const wick_hip_model *m, const wick_hip_kv *kv, int start, int t
 
 // Several tokens run their products on the matrix cores (gemm_kernel), except 2 or
 // 3 of a small model, which stream the weights through gemv_kernel in one pass:
-// the whole forward took 0.96 / 1.03 ms against 1.13 / 1.07 ms at hidden 576, but
+// the whole forward took 0.91 / 0.97 ms against 0.96 / 0.96 ms at hidden 576, but
 // 298 / 275 us against 259 / 235 us at hidden 2048.
 bool products_on_mfma(const wick_hip_model_config &c, int t) { return t >= 4 || (t > 1 && c.hidden > 1024); }
 
 // One product with a fused epilogue: g.norm (optional) is the RMSNorm a GEMV
-// applies to its input rows; the GEMM takes it split (GemvArgs::ssq).
-int product(wick_hip_model *m, int epi, const wick::GemvArgs &g, bool gemm, const char *what) {
+// applies to its input rows; the GEMM takes it split (GemmArgs::ssq).
+int product(wick_hip_model *m, int epi, const wick::GemmArgs &g, bool gemm, const char *what) {
     const hipError_t e = gemm ? wick::launch_gemm(epi, g, m->stream) : wick::launch_gemv(epi, g, m->stream);
     if (e != hipSuccess) return hip_fail(e, what);
     return WICK_HIP_OK;
@@ -218,7 +219,7 @@ int forward_device(wick_hip_model *m, wick_hip_kv *kv, const uint32_t *tok_dev, 
                                           m->layers[0].attn_norm, m->ssq);
         if (e != hipSuccess) return hip_fail(e, "embed kernel launch");
     }
-    const auto normed = [&](wick::GemvArgs &g, const float *norm) {
+    const auto normed = [&](wick::GemmArgs &g, const float *norm) {
         g.eps = c.rms_eps;
         if (gemm) {
             g.x = m->xg;
@@ -229,7 +230,7 @@ int forward_device(wick_hip_model *m, wick_hip_kv *kv, const uint32_t *tok_dev, 
             g.norm = norm;
         }
     };
-    const auto next_norm = [&](wick::GemvArgs &g, const float *norm) {
+    const auto next_norm = [&](wick::GemmArgs &g, const float *norm) {
         if (!gemm) return;
         g.xg = m->xg;
         g.xnorm = norm;
@@ -243,7 +244,7 @@ int forward_device(wick_hip_model *m, wick_hip_kv *kv, const uint32_t *tok_dev, 
                          c.hidden <= 2048;
     for (int li = 0; li < c.layers; li++) {
         const wick_hip_model::Layer &L = m->layers[li];
-        wick::GemvArgs g{};
+        wick::GemmArgs g{};
         normed(g, L.attn_norm);
         g.w = L.wqkv;
         g.out0 = m->q;
@@ -267,7 +268,7 @@ int forward_device(wick_hip_model *m, wick_hip_kv *kv, const uint32_t *tok_dev, 
                                   : 1;
         if (fused < 0) return fused;
         if (fused == 0) {
-            g = wick::GemvArgs{};
+            g = wick::GemmArgs{};
             g.x = m->x;
             g.parts = m->oparts;
             g.nparts = units;
@@ -283,7 +284,7 @@ int forward_device(wick_hip_model *m, wick_hip_kv *kv, const uint32_t *tok_dev, 
             g.t = 1;
             RC_TRY(product(m, wick::kEpiSwiglu, g, false, "residual + gate/up product launch"));
 
-            g = wick::GemvArgs{};
+            g = wick::GemmArgs{};
             g.x = m->h;
             g.w = L.w_down;
             g.resid = m->xr;
@@ -296,9 +297,18 @@ int forward_device(wick_hip_model *m, wick_hip_kv *kv, const uint32_t *tok_dev, 
             continue;
         }
 
-        RC_TRY(wick::attend_model(kv, li, c.heads, m->q, m->k, m->v, t, start, m->att, counters ? counters + 1 : nullptr));
+        // One token over a longer cache: the o product merges the chunks'
+        // states itself where those are few (one launch less).
+        wick::DecodeStates states{};
+        const int split = t == 1 ? wick::attend_model_states(kv, li, c.heads, m->q, m->k, m->v, start, &states,
+                                                             counters ? counters + 1 : nullptr)
+                                 : 1;
+        if (split < 0) return split;
+        if (split != 0)
+            RC_TRY(wick::attend_model(kv, li, c.heads, m->q, m->k, m->v, t, start, m->att,
+                                      counters ? counters + 1 : nullptr));
 
-        g = wick::GemvArgs{};
+        g = wick::GemmArgs{};
         g.x = m->att;
         g.w = L.wo;
         g.out0 = m->x;
@@ -307,9 +317,14 @@ int forward_device(wick_hip_model *m, wick_hip_kv *kv, const uint32_t *tok_dev, 
         g.cols = m->qd;
         g.t = t;
         next_norm(g, L.ffn_norm);
-        RC_TRY(product(m, wick::kEpiResid, g, gemm, "o product launch"));
+        if (split == 0) {
+            const hipError_t e = wick::launch_gemv_states(g, states, s);
+            if (e != hipSuccess) return hip_fail(e, "o product launch");
+        } else {
+            RC_TRY(product(m, wick::kEpiResid, g, gemm, "o product launch"));
+        }
 
-        g = wick::GemvArgs{};
+        g = wick::GemmArgs{};
         normed(g, L.ffn_norm);
         g.w = L.w_gate;
         g.w2 = L.w_up;
@@ -320,7 +335,7 @@ int forward_device(wick_hip_model *m, wick_hip_kv *kv, const uint32_t *tok_dev, 
         g.t = t;
         RC_TRY(product(m, wick::kEpiSwiglu, g, gemm, "gate/up product launch"));
 
-        g = wick::GemvArgs{};
+        g = wick::GemmArgs{};
         g.x = m->h;
         g.w = L.w_down;
         g.out0 = m->x;
@@ -331,7 +346,7 @@ int forward_device(wick_hip_model *m, wick_hip_kv *kv, const uint32_t *tok_dev, 
         next_norm(g, li + 1 < c.layers ? m->layers[li + 1].attn_norm : m->norm);
         RC_TRY(product(m, wick::kEpiResid, g, gemm, "down product launch"));
     }
-    wick::GemvArgs g{};
+    wick::GemmArgs g{};
     if (all_logits) {
         normed(g, m->norm);
     } else {

@@ -25,6 +25,24 @@ constexpr int kMaxParts = 4;
 constexpr int kArgmaxRows = 4;
 __host__ __device__ inline int argmax_parts(int rows) { return (rows + kArgmaxRows - 1) / kArgmaxRows; }
 
+// The states of a split single-token decode, before their merge: chunk c of head
+// h = kvh * group + hh at ((kvh * hslices + hh / 16) * 16 + hh % 16) * stride + c
+// in m (log2 units), l and, times head_dim, o.
+struct DecodeStates {
+    const float *o, *m, *l;
+    int head_dim, group, hslices, stride, nchunks;
+};
+
+// Most chunks the o product merges itself, and the most columns it then has:
+// every one of its workgroups reads all the states (16 of 576 columns are 37 KB)
+// in place of a merge launch.  Decoding SmolLM2-135M at 200 / 300 / 500 / 900
+// positions (4, 5, 8, 15 chunks) 589 -> 534, 606 -> 571, 612 -> 592, 626 -> 614
+// us a token, the Qwen2.5-0.5B size 693 -> 646, 678 -> 646, 679 -> 661, 700 ->
+// 681; 16 longer chunks in place of more gained nothing (1500 positions 626 ->
+// 633, 3000 631 -> 664).
+constexpr int kStateChunks = 16;
+constexpr int kStateCols = 1024;
+
 struct GemvArgs {
     const float *x;       // input rows [t][cols]
     const float *norm;    // RMSNorm weight [cols] applied to each input row first, or null
@@ -44,11 +62,14 @@ struct GemvArgs {
     float *xout;
     // kEpiResid: the value added to, resid[tok][row] (stride ld0); null: out0 itself
     const float *resid;
-    // launch_gemm: RMSNorm split over two products.  A kEpiResid product with
-    // xg also writes out0 * xnorm (the next norm's weight) to xg and, per token,
-    // each 16-row block's sum of squares to xssq[block][t]; the product that
-    // reads xg gets those sums as ssq (nssq blocks, added in order) and applies
-    // the norm's factor 1/sqrt(sum/cols + eps) to its own sums.
+};
+
+// launch_gemm's: RMSNorm split over two products.  A kEpiResid product with xg
+// also writes out0 * xnorm (the next norm's weight) to xg and, per token, each
+// 16-row block's sum of squares to xssq[block][t]; the product that reads xg
+// gets those sums as ssq (nssq blocks, added in order) and applies the norm's
+// factor 1/sqrt(sum/cols + eps) to its own sums.
+struct GemmArgs : GemvArgs {
     const float *ssq;
     int nssq;
     float *xg, *xssq;
@@ -59,9 +80,13 @@ struct GemvArgs {
 // epilogue `epi`; t tokens, cols % 4 == 0.
 hipError_t launch_gemv(int epi, const GemvArgs &a, hipStream_t s);
 
+// The kEpiResid product of one token whose input row is the attention output
+// that st's states merge to (a.x is not read); cols <= kStateCols.
+hipError_t launch_gemv_states(const GemvArgs &a, const DecodeStates &st, hipStream_t s);
+
 // The same products for several tokens on the matrix cores (a.norm must be
-// null, see GemvArgs::ssq; kEpiQkv: splits and rows multiples of 16).
-hipError_t launch_gemm(int epi, const GemvArgs &a, hipStream_t s);
+// null; kEpiQkv: splits and rows multiples of 16).
+hipError_t launch_gemm(int epi, const GemmArgs &a, hipStream_t s);
 
 // x[i][:] = embed[tokens[i]][:] for i < t (token ids already validated).
 // step: when non-null, the token of row i is tokens[*step + i] (device counter).
