@@ -534,3 +534,34 @@ def test_o_product_merges_the_chunks(heads, kvh, n):
         cache.len = 0
         first = m.prefill(cache, prompt)
         assert [first] + m.decode(cache, first, 59) == ids
+
+
+@pytest.mark.parametrize("hidden,ff,vocab", [
+    (2052, 2050 * 4, 2100),   # every product on the long-row kernel: 4 columns past a pass, rows left over
+    (2304, 14336, 4099),      # its longest row, a head whose last pair is short
+    (2304, 14340, 2048),      # one past it
+    (4096, 1028, 1024),       # whole passes; a down product too narrow for it
+])
+def test_single_token_products_on_long_rows(hidden, ff, vocab):
+    """One-token forwards whose rows are too long for one pass: logits of 4 steps within 1e-4
+    of the CPU oracle and the same greedy ids.  Weights N(0, 1/hidden), so products of unit-rms
+    rows are of order 1 and two orders of a sum of n terms differ by about sqrt(n) 2^-24,
+    at most 8e-6 here."""
+    cfg = Config("llama", hidden, ff, 1, 4, 2, 64, vocab, rms_eps=1e-5, rope_theta=10000.0, tie_embeddings=True)
+    w = random_weights(cfg, seed=hidden, std=hidden ** -0.5)
+    rng = np.random.default_rng(ff)
+    w["norm"] = (1 + 0.2 * rng.standard_normal(hidden)).astype(np.float32)
+    w["layers"][0]["ffn_norm"] = (1 + 0.2 * rng.standard_normal(hidden)).astype(np.float32)
+    om = ol.OracleModel(cfg, w)
+    st = om.new_state(8)
+    with DeviceModel(cfg, w) as m:
+        cache = m.new_cache(8)
+        tok, ids = 5, []
+        for _ in range(4):
+            want = om.forward(st, [tok])
+            got = m.forward(cache, [tok])
+            assert np.abs(got - want).max() < 1e-4
+            tok = ol.argmax(want[0])
+            ids.append(tok)
+        cache.len = 0
+        assert m.decode(cache, 5, 4) == ids

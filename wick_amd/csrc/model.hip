@@ -13,6 +13,8 @@
 
 #include <math.h>
 
+#include <algorithm>
+
 #include "model_kernels.h"
 #include "wave_ops.h"
 
@@ -317,6 +319,132 @@ __global__ __launch_bounds__(256) void gemv1_kernel(const GemvArgs a) {
                 if (row0 + r < a.rows) arg_better(acc[r], row0 + r, bv, bi);
             reinterpret_cast<float2 *>(a.out1)[row0 / R] = make_float2(bv, __int_as_float(bi));
         }
+    }
+}
+
+// One token, rows too long for gemv1_kernel: HBM-bound, and gemv_kernel's waves
+// each read the input row again for every row of weights (twice with a norm)
+// through the L1 that the weights come through.  Here a workgroup stages the
+// row in LDS once, times the norm's weight (its factor multiplies the sums), and
+// its waves stream R rows of weights after R rows, the next U float4s of each
+// requested while these are multiplied, across row ends too.  A layer of 4096 x
+// 14336 (8B size): q/k/v 23.4 -> 17.8 us, gate/up 79.4 -> 69.5 (6.8 TB/s), down
+// 38.7 -> 37.0; a head of 32000 rows 95.4 -> 91.4.
+constexpr int kWideWaves = 8;
+
+template <int R, int U, int EPI, bool NORM>
+__global__ __launch_bounds__(64 * kWideWaves) void gemv_wide_kernel(const GemvArgs a) {
+    static_assert(EPI != kEpiArgmax || R == kArgmaxRows, "one pair per kArgmaxRows rows");
+    constexpr int M = EPI == kEpiSwiglu ? 2 : 1, NW = kWideWaves;
+    extern __shared__ f4 sx[];  // the row, zero-padded to whole passes
+    __shared__ float sss[NW];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int C4 = a.cols >> 2, passes = (C4 + 64 * U - 1) / (64 * U);
+    const int groups = (a.rows + R - 1) / R, step = gridDim.x * NW;
+    const f4 zero = {0.f, 0.f, 0.f, 0.f};
+    f4 wv[2][M][R][U];
+    const auto load = [&](f4 (&b)[M][R][U], int g, int p) {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const size_t row = (size_t)min(g * R + r, a.rows - 1) * a.cols;
+            const f4 *W = reinterpret_cast<const f4 *>(a.w + row);
+            const f4 *W2 = reinterpret_cast<const f4 *>((M == 2 ? a.w2 : a.w) + row);
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int c = min(64 * (p * U + u) + lane, C4 - 1);
+                b[0][r][u] = __builtin_nontemporal_load(W + c);
+                if (M == 2) b[M - 1][r][u] = __builtin_nontemporal_load(W2 + c);
+            }
+        }
+    };
+    int g = blockIdx.x * NW + w, p = 0;
+    load(wv[0], min(g, groups - 1), 0);
+    float ss = 0.f;
+    for (int c = threadIdx.x; c < passes * 64 * U; c += 64 * NW) {
+        f4 x = c < C4 ? reinterpret_cast<const f4 *>(a.x)[c] : zero;
+        if (NORM) {
+            ss = dot4(x, x, ss);
+            x = c < C4 ? x * reinterpret_cast<const f4 *>(a.norm)[c] : zero;
+        }
+        sx[c] = x;
+    }
+    if (NORM) {
+        ss = wave_sum(ss);
+        if (lane == 0) sss[w] = ss;
+    }
+    __syncthreads();
+    float scale = 1.f;
+    if (NORM) {
+        ss = 0.f;
+#pragma unroll
+        for (int j = 0; j < NW; j++) ss += sss[j];
+        scale = 1.0f / sqrtf(ss / (float)a.cols + a.eps);
+    }
+    float acc[M][R];
+#pragma unroll
+    for (int m = 0; m < M; m++)
+#pragma unroll
+        for (int r = 0; r < R; r++) acc[m][r] = 0.f;
+    // this batch's products while the next one's weights (the row's next pass, or
+    // the next row's first) are on their way
+    const auto turn = [&](f4 (&b)[M][R][U], f4 (&next)[M][R][U]) {
+        const bool last = p + 1 == passes;
+        const int ng = last ? g + step : g, np = last ? 0 : p + 1;
+        load(next, min(ng, groups - 1), np);
+        __builtin_amdgcn_sched_barrier(0);
+        const bool tail = 64 * U * (p + 1) > C4;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int c = 64 * (p * U + u) + lane;
+            const f4 x = sx[c];
+#pragma unroll
+            for (int m = 0; m < M; m++)
+#pragma unroll
+                for (int r = 0; r < R; r++) acc[m][r] = dot4(tail && c >= C4 ? zero : b[m][r][u], x, acc[m][r]);
+        }
+        if (last) {
+#pragma unroll
+            for (int m = 0; m < M; m++)
+#pragma unroll
+                for (int r = 0; r < R; r++) acc[m][r] = wave_sum(acc[m][r]) * scale;
+            if (lane == 0) {
+                float bv = -INFINITY;
+                int bi = 0x7fffffff;
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    const int row = g * R + r;
+                    if (row >= a.rows) break;
+                    const float d = acc[0][r];
+                    if (EPI == kEpiStore || EPI == kEpiArgmax) {
+                        a.out0[row] = d;
+                    } else if (EPI == kEpiResid) {
+                        a.out0[row] = (a.resid ? a.resid : a.out0)[row] + d;
+                    } else if (EPI == kEpiQkv) {
+                        if (row < a.split0)
+                            a.out0[row] = d;
+                        else if (row < a.split1)
+                            a.out1[row - a.split0] = d;
+                        else
+                            a.out2[row - a.split1] = d;
+                    } else {  // silu_mul: g / (1 + exp(-g)) * u
+                        a.out0[row] = d / (1.0f + expf(-d)) * acc[M - 1][r];
+                    }
+                    if (EPI == kEpiArgmax) arg_better(d, row, bv, bi);
+                }
+                if (EPI == kEpiArgmax) reinterpret_cast<float2 *>(a.out1)[g] = make_float2(bv, __int_as_float(bi));
+            }
+#pragma unroll
+            for (int m = 0; m < M; m++)
+#pragma unroll
+                for (int r = 0; r < R; r++) acc[m][r] = 0.f;
+        }
+        g = ng;
+        p = np;
+    };
+    while (g < groups) {
+        turn(wv[0], wv[1]);
+        if (g >= groups) break;
+        turn(wv[1], wv[0]);
     }
 }
 
@@ -825,6 +953,27 @@ hipError_t gemv1_launch(const GemvArgs &a, hipStream_t s) {
     return hipErrorInvalidValue;
 }
 
+// Where gemv_wide_kernel is the faster one: 16 MB of weights or more (the head
+// at 1001 x 2052: 7.9 against 9.3 us), the row (padded to passes of 2048 columns)
+// and the waves' sums within 64 KiB of LDS, and either a norm (gemv_kernel then
+// reads the input row twice) or rows of 8192 columns and more (2048 x 5632: 9.6
+// against 9.9 us; 4096 x 4096 equal).
+bool gemv_wide(const GemvArgs &a) {
+    return (long long)a.rows * a.cols >= (4 << 20) && a.cols <= 7 * 2048 && (a.norm ? a.cols > 2048 : a.cols >= 8192);
+}
+
+template <int R, int U, int EPI>
+hipError_t gemv_wide_launch(const GemvArgs &a, hipStream_t s) {
+    const int groups = (a.rows + R - 1) / R, passes = ((a.cols >> 2) + 64 * U - 1) / (64 * U);
+    const dim3 grid((unsigned)std::min((groups + kWideWaves - 1) / kWideWaves, 512)), block(64 * kWideWaves);
+    const size_t lds = (size_t)passes * 64 * U * sizeof(f4);
+    if (a.norm)
+        hipLaunchKernelGGL((gemv_wide_kernel<R, U, EPI, true>), grid, block, lds, s, a);
+    else
+        hipLaunchKernelGGL((gemv_wide_kernel<R, U, EPI, false>), grid, block, lds, s, a);
+    return hipGetLastError();
+}
+
 // One token: one row per wave (the LM head, kEpiStore / kEpiArgmax, 4 rows per
 // wave to keep more of its 100+ MB in flight per wave), the input row through
 // LDS when it fits one pass (64 * 8 float4s), else gemv_kernel.  Several
@@ -835,13 +984,16 @@ hipError_t gemv_epi(const GemvArgs &a, hipStream_t s) {
     if constexpr (EPI == kEpiArgmax) {
         if (a.t != 1 || !a.out1) return hipErrorInvalidValue;
         if (a.cols <= 4 * 64 * 4) return gemv1_launch<kArgmaxRows, EPI>(a, s);
+        if (gemv_wide(a)) return gemv_wide_launch<kArgmaxRows, 2, EPI>(a, s);
         return gemv_launch<1, kArgmaxRows, 4, EPI>(a, s);
     } else {
         if (a.t > 1) return gemv_launch<4, 1, 4, EPI>(a, s);
         if constexpr (EPI == kEpiStore) {
             if (a.cols <= 4 * 64 * 4) return gemv1_launch<4, EPI>(a, s);
+            if (gemv_wide(a)) return gemv_wide_launch<4, 2, EPI>(a, s);
             return gemv_launch<1, 4, 4, EPI>(a, s);
         }
+        if (gemv_wide(a)) return gemv_wide_launch<1, EPI == kEpiSwiglu ? 4 : 8, EPI>(a, s);
         if (one_pass) return gemv1_launch<1, EPI>(a, s);
         return gemv_launch<1, 1, 8, EPI>(a, s);
     }
