@@ -120,6 +120,34 @@ def test_sort_over_many_workgroups(vocab, top_k):
             assert ds.rng_state() == os_.rng.state()
 
 
+@pytest.mark.parametrize("vocab,top_k", [(70, 64), (4096, 40), (4097, 64), (49152, 1), (49152, 40), (65537, 16),
+                                         (65537, 17), (196608, 64)])
+def test_top_k_behind_a_loose_bound(vocab, top_k):
+    """The top-k taken per slice behind a bound from its waves, then from the slices: one and
+    two ids a wave, a slice of two ids, the longest slices; and logits whose bound is loose
+    (the best ids all in one slice or in one wave, hundreds of equal ones), infinite and NaN."""
+    rng = np.random.default_rng(vocab + top_k)
+    cfg = SamplerConfig(temperature=0.9, top_k=top_k, top_p=0.95, seed=3)
+    with DeviceSampler(cfg, vocab) as ds:
+        os_ = ol.OracleSampler(cfg)
+        for kind in ("normal", "falling", "rising", "wave", "equal", "-inf", "all -inf", "+inf", "-nan"):
+            x = logits_of("normal", vocab, rng)
+            at = rng.integers(0, vocab, 5)
+            if kind in ("falling", "rising"):
+                x = np.sort(x)[::-1 if kind == "falling" else 1].copy()
+            elif kind == "wave":  # ids 64..127 of every 1024: one wave's in its slice
+                x[np.arange(vocab) // 64 % 16 == 1] += 20
+            elif kind == "equal":
+                x[vocab // 3:vocab // 3 + 400] = 15.0
+            elif kind == "all -inf":
+                x[:] = -np.inf
+            elif kind != "normal":
+                x[at] = {"+inf": np.inf, "-inf": -np.inf, "-nan": np.float32(np.copysign(np.nan, -1.0))}[kind]
+            with np.errstate(invalid="ignore"):
+                check_draw(ds, os_, x, np.zeros(0, np.uint32), f"{vocab}/{top_k}/{kind}")
+        assert ds.rng_state() == os_.rng.state()
+
+
 def test_reference_unit_cases_on_device():
     """src/sampler.rs:150-171 through the device sampler."""
     logits = np.array([0.0, 3.0, 1.0, 2.9], np.float32)

@@ -44,6 +44,7 @@ constexpr int kMaxBins = 2048;         // 11-bit digits
 constexpr int kList = 4096;            // largest candidate set sorted in LDS
 constexpr int kSlicePer = kSliceMax / kT;  // slice entries per thread in the split kernel
 constexpr int kPartCand = 1024;        // candidates one slice may hold at its k-th key
+constexpr int kQuickCand = 256;        // candidates placed by rank behind quick_bound; past these a radix select is cheaper
 
 typedef float f4 __attribute__((ext_vector_type(4)));
 
@@ -260,14 +261,39 @@ __device__ __forceinline__ int draw_index(const float *p, int keep, float r, boo
     return keep - 1;
 }
 
-// Bitonic sort of one key per lane, ascending with the lane index.
+// Bitonic sort of one key per lane, ascending with the lane index.  The partner
+// at a stride of 1 to 8 lanes comes by DPP, at 16 and 32 as the pair of a
+// permlane swap, whose order does not matter to min and max: the 21 steps wait
+// for no LDS (figures at quick_bound).
 __device__ __forceinline__ unsigned long long wave_sort(unsigned long long v) {
     const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int size = 2; size <= 64; size <<= 1) {
 #pragma unroll
         for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            const uint32_t lo = __shfl_xor((uint32_t)v, stride, 64), hi = __shfl_xor((uint32_t)(v >> 32), stride, 64);
+            const uint32_t vl = (uint32_t)v, vh = (uint32_t)(v >> 32);
+            uint32_t lo, hi;
+            if (stride >= 16) {
+                const auto pl = stride == 16 ? __builtin_amdgcn_permlane16_swap(vl, vl, false, false)
+                                             : __builtin_amdgcn_permlane32_swap(vl, vl, false, false);
+                const auto ph = stride == 16 ? __builtin_amdgcn_permlane16_swap(vh, vh, false, false)
+                                             : __builtin_amdgcn_permlane32_swap(vh, vh, false, false);
+                v = ((unsigned long long)ph[0] << 32) | pl[0];
+                lo = pl[1];
+                hi = ph[1];
+            } else if (stride == 8) {
+                lo = dpp_i<kDppRowRor8>(vl);
+                hi = dpp_i<kDppRowRor8>(vh);
+            } else if (stride == 4) {  // lane ^ 7, then ^ 3
+                lo = dpp_i<kDppQuadXor3>(dpp_i<kDppRowHalfMirror>(vl));
+                hi = dpp_i<kDppQuadXor3>(dpp_i<kDppRowHalfMirror>(vh));
+            } else if (stride == 2) {
+                lo = dpp_i<kDppQuadXor2>(vl);
+                hi = dpp_i<kDppQuadXor2>(vh);
+            } else {
+                lo = dpp_i<kDppQuadXor1>(vl);
+                hi = dpp_i<kDppQuadXor1>(vh);
+            }
             const unsigned long long o = ((unsigned long long)hi << 32) | lo;
             const bool keep_min = ((lane & stride) == 0) == ((lane & size) == 0);
             v = keep_min ? (v < o ? v : o) : (v < o ? o : v);
@@ -462,6 +488,30 @@ __host__ __device__ inline uint32_t top_k_of(const SampleArgs &a) {
     return (a.top_k == 0u || a.top_k > (uint32_t)a.vocab) ? (uint32_t)a.vocab : a.top_k;
 }
 
+// A bound with at least k of the block's keys at or below it, so the k best are
+// among those: every wave's ceil(k / kW)-th smallest of its lanes' smallest keys
+// (`least`; ~0 for none), the largest of these over the waves.  A tight one needs
+// the radix select, whose digits cost seven barriers and an LDS histogram each;
+// this costs one barrier and leaves a few times k candidates to be ranked.  With
+// the slices merged behind the same kind of bound and wave_sort off LDS, one draw
+// with top-k 40 over 32000 ids 19.1 -> 13.6 us, 49152 18.4 -> 14.1, 151936 20.3 ->
+// 15.8; top-k 50 over 128256 20.7 -> 17.5.  Sets s.count to 0.
+__device__ __forceinline__ uint32_t quick_bound(uint32_t least, uint32_t k, SampleLds &s) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    uint32_t b = 0u;
+    for (uint32_t r = 0; r < (k + kW - 1) / kW; r++) {
+        b = wave_min(least);
+        if (lane == __builtin_ctzll(__ballot(least == b))) least = 0xffffffffu;
+    }
+    if (lane == 0) s.wsum[w] = b;
+    if (threadIdx.x == 0) s.count = 0u;
+    __syncthreads();
+    b = s.wsum[0];
+#pragma unroll
+    for (int j = 1; j < kW; j++) b = max(b, s.wsum[j]);
+    return b;
+}
+
 // The first kernel of a draw: workgroup g owns the slice [g * slice, +slice)
 // of the vocabulary (slices are whole bitset words).  It applies the
 // repetition penalty to its ids (src/sampler.rs:75-83, each distinct id once),
@@ -503,36 +553,46 @@ __global__ __launch_bounds__(kT) void sample_split_kernel(SampleArgs a) {
     }
     const uint32_t k = top_k_of(a);
     if (!a.split_top_k || k > (uint32_t)kFastK) return;
-    uint32_t key[kSlicePer];
+    uint32_t key[kSlicePer], least = 0xffffffffu;
 #pragma unroll
     for (int j = 0; j < kSlicePer; j++) {
         const int i = lo + j * kT + tid;
-        key[j] = i < hi ? desc_key(x[i]) : 0u;
+        key[j] = i < hi ? desc_key(x[i]) : 0xffffffffu;
+        least = min(least, key[j]);
     }
-    uint32_t bound = 0xffffffffu, nset = (uint32_t)(hi - lo);
-    if (k < nset)
-        nset = select_bound<8, 8, 8, 8>(
-            [&](auto &&f) {
+    auto gather = [&](uint32_t bound) {
 #pragma unroll
-                for (int j = 0; j < kSlicePer; j++)
-                    if (lo + j * kT + tid < hi) f(key[j]);
-            },
-            k, 64u, s, &bound);
-    if (tid == 0) s.count = 0u;
-    __syncthreads();
-    if (nset > (uint32_t)kPartCand) {  // too many ties: the final kernel takes the whole vocabulary
-        if (tid == 0) a.part_count[g] = -1;
-        return;
-    }
-#pragma unroll
-    for (int j = 0; j < kSlicePer; j++) {
-        const int i = lo + j * kT + tid;
-        if (i < hi && key[j] <= bound) {
-            const uint32_t pos = atomicAdd(&s.count, 1u);
-            if (pos < (uint32_t)kPartCand) s.l.cand[pos] = ((unsigned long long)key[j] << 32) | (uint32_t)i;
+        for (int j = 0; j < kSlicePer; j++) {
+            const int i = lo + j * kT + tid;
+            if (i < hi && key[j] <= bound) {
+                const uint32_t pos = atomicAdd(&s.count, 1u);
+                if (pos < (uint32_t)kPartCand) s.l.cand[pos] = ((unsigned long long)key[j] << 32) | (uint32_t)i;
+            }
         }
+        __syncthreads();
+    };
+    gather(quick_bound(least, k, s));
+    uint32_t nset = s.count;
+    if (nset > (uint32_t)kQuickCand) {  // many ties, or a few waves hold the best ids
+        __syncthreads();
+        uint32_t bound = 0xffffffffu;
+        nset = (uint32_t)(hi - lo);
+        if (k < nset)
+            nset = select_bound<8, 8, 8, 8>(
+                [&](auto &&f) {
+#pragma unroll
+                    for (int j = 0; j < kSlicePer; j++)
+                        if (lo + j * kT + tid < hi) f(key[j]);
+                },
+                k, 64u, s, &bound);
+        if (tid == 0) s.count = 0u;
+        __syncthreads();
+        if (nset > (uint32_t)kPartCand) {  // too many ties: the final kernel takes the whole vocabulary
+            if (tid == 0) a.part_count[g] = -1;
+            return;
+        }
+        gather(bound);
     }
-    __syncthreads();
     const int n = (int)min(s.count, (uint32_t)kPartCand);
     if (n <= 64) {  // one wave sorts them
         if (tid < 64) {
@@ -589,9 +649,8 @@ __global__ __launch_bounds__(kT) void sample_kernel(SampleArgs a) {
     const bool fast = s.fast != 0;
     bool in_lds = true;
     if (fast) {
-        // Each thread holds at most one of the slices' pairs; a radix select on
-        // their keys bounds the k best, and one wave sorts the (usually few)
-        // pairs up to that bound -- more are placed by rank.
+        // Each thread holds at most one of the slices' pairs; those up to a bound
+        // are sorted by one wave, or placed by rank where they are more.
         const int slots = a.parts * kFastK;
         unsigned long long mine = ~0ull;
         bool have = false;
@@ -600,12 +659,25 @@ __global__ __launch_bounds__(kT) void sample_kernel(SampleArgs a) {
             have = tid - g * kFastK < min(s.pcount[g], kFastK);
             if (have) mine = a.part_cand[tid];
         }
-        const uint32_t total = (uint32_t)__syncthreads_count(have);
-        uint32_t bound = 0xffffffffu;
-        if (k < total)
-            select_bound<8, 8, 8, 8>([&](auto &&f) { if (have) f((uint32_t)(mine >> 32)); }, k, 64u, s, &bound);
+        // every slice's ceil(k / parts)-th best, the largest of these: at least k
+        // pairs up to it, where every slice has as many
+        const int q = ((int)k + a.parts - 1) / a.parts - 1;
+        uint32_t b = 0u;
+        if (lane < a.parts)
+            b = q < s.pcount[lane] ? (uint32_t)(a.part_cand[lane * kFastK + q] >> 32) : 0xffffffffu;
+        uint32_t bound = ~wave_min(~b);
         if (have && (uint32_t)(mine >> 32) <= bound) s.l.cand[atomicAdd(&s.count, 1u)] = mine;
         __syncthreads();
+        if (s.count > (uint32_t)kQuickCand) {  // a few slices hold the best ids
+            const uint32_t total = (uint32_t)__syncthreads_count(have);
+            bound = 0xffffffffu;
+            if (k < total)
+                select_bound<8, 8, 8, 8>([&](auto &&f) { if (have) f((uint32_t)(mine >> 32)); }, k, 64u, s, &bound);
+            if (tid == 0) s.count = 0u;
+            __syncthreads();
+            if (have && (uint32_t)(mine >> 32) <= bound) s.l.cand[atomicAdd(&s.count, 1u)] = mine;
+            __syncthreads();
+        }
         const int n = (int)s.count;
         if (n < (int)k && tid == 0) s.bad = 4;
         if (n <= 64) {

@@ -15,6 +15,8 @@ namespace wick {
 
 constexpr int kDppQuadXor1 = 0xB1;       // quad_perm [1, 0, 3, 2]
 constexpr int kDppQuadXor2 = 0x4E;       // quad_perm [2, 3, 0, 1]
+constexpr int kDppQuadXor3 = 0x1B;       // quad_perm [3, 2, 1, 0]
+constexpr int kDppRowRor8 = 0x128;       // lane i <- lane i ^ 8 within 16
 constexpr int kDppRowShr1 = 0x111;       // lane i <- lane i - 1 within 16
 constexpr int kDppRowHalfMirror = 0x141;  // lane i <- lane 7 - i within 8
 constexpr int kDppRowMirror = 0x140;      // lane i <- lane 15 - i within 16
@@ -50,6 +52,18 @@ __device__ __forceinline__ float wave_max(float v) {
     v = fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
     p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
+}
+
+// Minimum over the 64 lanes, in every lane.
+__device__ __forceinline__ unsigned wave_min(unsigned v) {
+    v = min(v, (unsigned)dpp_i<kDppQuadXor1>((int)v));
+    v = min(v, (unsigned)dpp_i<kDppQuadXor2>((int)v));
+    v = min(v, (unsigned)dpp_i<kDppRowHalfMirror>((int)v));
+    v = min(v, (unsigned)dpp_i<kDppRowMirror>((int)v));
+    auto p = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    v = min((unsigned)p[0], (unsigned)p[1]);
+    p = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return min((unsigned)p[0], (unsigned)p[1]);
 }
 
 // Sum of the 4 lanes l, l^16, l^32, l^48 (the same column of every row of 16).
