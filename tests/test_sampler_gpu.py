@@ -120,6 +120,24 @@ def test_sort_over_many_workgroups(vocab, top_k):
             assert ds.rng_state() == os_.rng.state()
 
 
+@pytest.mark.parametrize("vocab", [4097, 20001])
+@pytest.mark.parametrize("top_p", [0.9, 1.0])
+def test_draw_that_starts_from_zero(vocab, top_p):
+    """A generator whose first output has 24 leading zero bits (one in 2^24): the draw's
+    remainder is 0 before its first subtraction, so its walk starts term by term, with no
+    barrier of its own behind the walk for top-p, and takes the most likely id."""
+    cfg = SamplerConfig(temperature=1.0, top_k=0, top_p=top_p, seed=15115159)
+    os_ = ol.OracleSampler(cfg)
+    s1 = os_.rng.state()[1]
+    assert ((s1 * 5 << 7 | (s1 * 5 & (1 << 64) - 1) >> 57) * 9 & (1 << 64) - 1) >> 40 == 0
+    with DeviceSampler(cfg, vocab) as ds:
+        x = logits_of("normal", vocab, np.random.default_rng(vocab))
+        check_draw(ds, os_, x.copy(), np.zeros(0, np.uint32), f"{vocab}/{top_p}")
+        os_ = ol.OracleSampler(cfg)
+        assert os_.sample(x.copy()) == int(x.argmax())
+        assert ds.rng_state() == os_.rng.state()
+
+
 @pytest.mark.parametrize("vocab,top_k", [(70, 64), (4096, 40), (4097, 64), (49152, 1), (49152, 40), (65537, 16),
                                          (65537, 17), (196608, 64)])
 def test_top_k_behind_a_loose_bound(vocab, top_k):

@@ -1148,13 +1148,14 @@ __device__ __forceinline__ float walk(const float *__restrict__ p, int n, float 
             __syncthreads();
             if (next < nw) {
                 acc = s.acc;
-                if (s.hit >= 0) {
-                    *hit = s.hit;
-                    return acc;
-                }
+                *hit = s.hit;
                 next++;
             }
-            __syncthreads();  // the next turn writes what was just read
+            // The next turn writes what was just read; so does the first turn of a
+            // next walk on the same LDS, before any other barrier where it starts
+            // from zero.
+            __syncthreads();
+            if (*hit >= 0) return acc;
         }
     }
     return acc;
