@@ -72,7 +72,12 @@ const char *wick_hip_last_error(void);
 /* As wick_hip_kv_append, with k_dev / v_dev device arrays [t][kv_heads*head_dim]. */
 int wick_hip_kv_append_device(wick_hip_kv *kv, int layer, int start, int t, const float *k_dev, const float *v_dev);
 
-/* As wick_hip_attention, with q_dev / att_dev device arrays [t][heads*head_dim]. */
+/* As wick_hip_attention, with q_dev / att_dev device arrays [t][heads*head_dim].
+ * A few tokens over many keys (t > 1) share each block of rows' keys over several
+ * workgroups, whose states the handle keeps in a workspace (up to 4.3 MB) that it
+ * makes at the first such call on a stream, for up to 4 streams.  Past those, under
+ * stream capture, and where there is no memory for it, the call uses no workspace
+ * and is slower; its result then differs by rounding. */
 int wick_hip_attention_device(wick_hip_kv *kv, int layer, int heads, const float *q_dev, int t, int start,
                               float *att_dev);
 
@@ -85,10 +90,9 @@ int wick_hip_attention_device(wick_hip_kv *kv, int layer, int heads, const float
  * handle's workspace: it needs kv_heads * ceil(group / 16) * 16 * 256 *
  * (head_dim + 2) floats, at most 8 Mi (e.g. up to 31 kv heads at head_dim 64
  * with group <= 16, or 15 at head_dim 128); a larger shape returns
- * WICK_HIP_EINVAL.  Prefill (t > 1) uses no workspace: it never splits a few
- * tokens' keys over workgroups, as wick_hip_attention_device does from the
- * first call that may allocate.  Every call on one GPU
- * shares that array, so calls that overlap on one GPU (other handles or
+ * WICK_HIP_EINVAL.  Prefill (t > 1) uses no workspace: it never shares a few
+ * tokens' keys over workgroups, as wick_hip_attention_device does.  Every call on
+ * one GPU shares that array, so calls that overlap on one GPU (other handles or
  * streams included) race: serialise them.  Asynchronous on the handle's
  * stream. */
 int wick_hip_attention_device_noalloc(wick_hip_kv *kv, int layer, int heads, const float *q_dev, int t, int start,

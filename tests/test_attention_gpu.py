@@ -524,7 +524,7 @@ def test_decode_hip_graph_replays_match_eager():
 def test_prefill_split_over_workgroups(t, start, heads, kv_heads, d):
     """A few tokens over many keys: the blocks' keys shared by several workgroups and
     merged, against the oracle and against the entry point that never splits; bit-stable;
-    and unsplit, without allocating, where the first call is captured into a graph."""
+    and unsplit, without allocating, where the call is captured into a graph."""
     import torch
     q, k, v = make_inputs(start, t, start, heads, kv_heads, d, theta=1e6)
     blocks = kv_heads * ((t * heads // kv_heads + 15) // 16)
@@ -554,3 +554,57 @@ def test_prefill_split_over_workgroups(t, start, heads, kv_heads, d):
     ok, mabs, mrel = within_tol(split, want)
     assert ok, (mabs, mrel)
     assert within_tol(split, unsplit)[0]
+
+
+def test_prefill_split_calls_on_several_streams():
+    """Split prefill calls of one handle on six streams at once, and replays of a captured
+    call next to them: each stream's states are its own (the first four split, the others
+    and the captured call use none), so every output has the bits of the call alone."""
+    import torch
+    t, start, heads, kv_heads, d, n = 37, 3001, 14, 2, 64, 6
+    _, k, v = make_inputs(81, t, start, heads, kv_heads, d)
+    blocks = kv_heads * ((t * heads // kv_heads + 15) // 16)
+    qs = [torch.from_numpy(make_inputs(82 + i, t, 0, heads, kv_heads, d)[0]).cuda() for i in range(n)]
+    outs = [torch.full_like(q, float("nan")) for q in qs]
+    split, unsplit = [torch.empty_like(q) for q in qs], [torch.empty_like(q) for q in qs]
+    replayed = torch.full_like(qs[0], float("nan"))
+    streams = [torch.cuda.Stream() for _ in range(n)]
+    torch.cuda.synchronize()
+    with DeviceKvCache(1, start + t, kv_heads, d) as kv:
+        kv.append(0, 0, k, v)
+        staged = kv.scratch_bytes()
+
+        def call(i, out):
+            kv.set_stream(streams[i].cuda_stream)
+            kv.attention_device(0, heads, qs[i].data_ptr(), t, start, out.data_ptr())
+
+        for i in range(n):  # one after another, all on the first stream
+            kv.set_stream(streams[0].cuda_stream)
+            kv.attention_device(0, heads, qs[i].data_ptr(), t, start, split[i].data_ptr())
+            assert kv.last_grid() > blocks
+            kv.attention_device_noalloc(0, heads, qs[i].data_ptr(), t, start, unsplit[i].data_ptr())
+            kv.synchronize()
+        one = kv.scratch_bytes() - staged
+        assert 0 < one < 4.4e6
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=streams[0]):
+            call(0, replayed)
+            assert kv.last_grid() == blocks, "a captured call would share the handle's states"
+        for i in range(1, n):  # the workspaces, before anything overlaps
+            call(i, outs[i])
+            assert (kv.last_grid() > blocks) == (i < 4)
+            torch.cuda.synchronize()
+        assert kv.scratch_bytes() - staged == 4 * one
+        for out in outs:
+            out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        for rep in range(10):
+            for i in range(n):
+                call(i, outs[i])
+                if i % 2:
+                    with torch.cuda.stream(streams[n - 1]):
+                        graph.replay()
+        torch.cuda.synchronize()
+    for i in range(n):
+        assert torch.equal(outs[i], split[i] if i < 4 else unsplit[i]), i
+    assert torch.equal(replayed, unsplit[0])

@@ -62,9 +62,13 @@ struct wick_hip_kv {
     // decode split-K workspace (partial softmax states of the chunks)
     float *part = nullptr;
     int ws_units = 0;
-    // split prefill workspace (kPrefillStates row states), made at first use and
-    // never moved
-    float *ppart = nullptr;
+    // split prefill workspaces (kPrefillStates row states each), one per stream that
+    // has launched such a call; made at first use and never moved
+    struct PrefillSpace {
+        hipStream_t stream = nullptr;
+        float *buf = nullptr;
+    };
+    PrefillSpace pspace[4];
     // whether the static workspace's address was found on this device
     hipError_t static_rc = hipErrorNotInitialized;
     // options
@@ -223,18 +227,30 @@ int plan_decode(wick_hip_kv *kv, int layer, int group, int len, const float *q_d
     return WICK_HIP_OK;
 }
 
-// The split prefill's workspace; null where it cannot be had (the stream is
-// being captured and it is not there yet, or no memory): the call then runs
-// unsplit, which needs none.
+// The split prefill's workspace for a call on the handle's stream.  A prefill
+// writes nothing but its own output otherwise, so calls on several streams and
+// replays of a captured one may overlap: every stream has its own states, and a
+// call under capture, whose replays may run next to anything, has none.  Null
+// there, past the streams that pspace has room for, and where there is no memory:
+// the call then runs unsplit.
 float *prefill_workspace(wick_hip_kv *kv) {
-    if (kv->ppart) return kv->ppart;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(kv->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) return nullptr;
-    if (hipMalloc(&kv->ppart, wick::kPrefillStates * (kv->head_dim + 2) * sizeof(float)) != hipSuccess) {
+    if (hipStreamIsCapturing(kv->stream, &st) != hipSuccess) {
         (void)hipGetLastError();
-        kv->ppart = nullptr;
+        return nullptr;
     }
-    return kv->ppart;
+    if (st != hipStreamCaptureStatusNone) return nullptr;
+    for (wick_hip_kv::PrefillSpace &p : kv->pspace) {
+        if (p.buf && p.stream == kv->stream) return p.buf;
+        if (p.buf) continue;
+        if (hipMalloc(&p.buf, wick::kPrefillStates * (kv->head_dim + 2) * sizeof(float)) != hipSuccess) {
+            (void)hipGetLastError();
+            p.buf = nullptr;
+        }
+        p.stream = kv->stream;
+        return p.buf;
+    }
+    return nullptr;
 }
 
 int run_attention(wick_hip_kv *kv, int layer, int heads, const float *q_dev, int t, int start, float *att_dev,
@@ -280,10 +296,11 @@ int run_attention(wick_hip_kv *kv, int layer, int heads, const float *q_dev, int
     // (the no-allocation entry point never splits: its static workspace is one
     // for all handles, and its prefill calls may overlap)
     const int splits = static_part ? 1 : wick::prefill_splits(D, kv->num_cus, a);
-    if (splits > 1 && prefill_workspace(kv)) {
+    float *const states = splits > 1 ? prefill_workspace(kv) : nullptr;
+    if (states) {
         a.splits = splits;
         a.rows32 = a.zigzag = 0;
-        a.po = kv->ppart;
+        a.po = states;
         a.pm = a.po + wick::kPrefillStates * D;
         a.pl = a.pm + wick::kPrefillStates;
     }
@@ -551,9 +568,11 @@ int wick_hip_kv_create(int layers, int capacity, int kv_heads, int head_dim, wic
 void wick_hip_kv_destroy(wick_hip_kv *kv) {
     if (!kv) return;
     if (kv->stream) (void)hipStreamSynchronize(kv->stream);
-    float *bufs[] = {kv->k, kv->v, kv->q_dev, kv->att_dev, kv->kst_dev, kv->vst_dev, kv->part, kv->ppart, kv->io_dev};
+    float *bufs[] = {kv->k, kv->v, kv->q_dev, kv->att_dev, kv->kst_dev, kv->vst_dev, kv->part, kv->io_dev};
     for (float *b : bufs)
         if (b) (void)hipFree(b);
+    for (auto &p : kv->pspace)
+        if (p.buf) (void)hipFree(p.buf);
     if (kv->io_host) (void)hipHostFree(kv->io_host);
     if (kv->rope_cos) (void)hipFree(kv->rope_cos);
     if (kv->rope_sin) (void)hipFree(kv->rope_sin);
@@ -600,7 +619,8 @@ long long wick_hip_kv_scratch_bytes(const wick_hip_kv *kv) {
     if (!kv) return 0;
     size_t floats = kv->q_cap + kv->att_cap + 2 * kv->kst_cap + kv->io_cap + kv->io_host_cap;
     if (kv->part) floats += wick::decode_workspace_floats(kv->ws_units, kv->head_dim);
-    if (kv->ppart) floats += wick::kPrefillStates * (kv->head_dim + 2);
+    for (const auto &p : kv->pspace)
+        if (p.buf) floats += wick::kPrefillStates * (kv->head_dim + 2);
     return (long long)(floats * sizeof(float));
 }
 

@@ -140,5 +140,5 @@ class DeviceKvCache:
         return self._lib.wick_hip_kv_last_grid(self.handle)
 
     def scratch_bytes(self):
-        """Staging and decode workspace bytes the handle has allocated so far."""
+        """Staging and attention workspace bytes the handle has allocated so far."""
         return int(self._lib.wick_hip_kv_scratch_bytes(self.handle))
