@@ -608,3 +608,29 @@ def test_prefill_split_calls_on_several_streams():
     for i in range(n):
         assert torch.equal(outs[i], split[i] if i < 4 else unsplit[i]), i
     assert torch.equal(replayed, unsplit[0])
+
+
+def test_prefill_split_next_to_a_capture_on_another_stream():
+    """A handle's first split prefill, which makes its workspace, while another stream is
+    being captured: the capture goes on, and the call splits and gives its result."""
+    import torch
+    t, start, heads, kv_heads, d = 37, 3001, 14, 2, 64
+    q, k, v = make_inputs(91, t, start, heads, kv_heads, d)
+    qd, x = torch.from_numpy(q).cuda(), torch.zeros(64, device="cuda")
+    out = torch.full_like(qd, float("nan"))
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with DeviceKvCache(1, start + t, kv_heads, d) as kv:  # launches on its own stream
+        kv.append(0, 0, k, v)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            x.add_(1)
+            kv.attention_device(0, heads, qd.data_ptr(), t, start, out.data_ptr())
+            assert kv.last_grid() > kv_heads * ((t * heads // kv_heads + 15) // 16)
+        kv.synchronize()
+        for _ in range(3):
+            graph.replay()
+        torch.cuda.synchronize()
+    assert x.eq(3).all()
+    want = ol.attention(q, k, v, t, start, heads, kv_heads, d)
+    assert within_tol(out.cpu().numpy(), want)[0]

@@ -243,7 +243,13 @@ float *prefill_workspace(wick_hip_kv *kv) {
     for (wick_hip_kv::PrefillSpace &p : kv->pspace) {
         if (p.buf && p.stream == kv->stream) return p.buf;
         if (p.buf) continue;
-        if (hipMalloc(&p.buf, wick::kPrefillStates * (kv->head_dim + 2) * sizeof(float)) != hipSuccess) {
+        // another stream may be in a capture, which an allocation in the default
+        // mode would end
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        const hipError_t ex = hipThreadExchangeStreamCaptureMode(&mode);
+        const hipError_t e = hipMalloc(&p.buf, wick::kPrefillStates * (kv->head_dim + 2) * sizeof(float));
+        if (ex == hipSuccess) (void)hipThreadExchangeStreamCaptureMode(&mode);
+        if (e != hipSuccess) {
             (void)hipGetLastError();
             p.buf = nullptr;
         }
