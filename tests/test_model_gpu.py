@@ -508,6 +508,24 @@ def test_products_of_several_tokens(hidden, ff, vocab, t):
     assert np.abs(again - alone).max() < 1e-4
 
 
+@pytest.mark.parametrize("t", [2, 17])
+def test_products_past_32_bit_row_offsets(t):
+    """A down product over rows of 2^22 + 4 columns, past the matrix-core products' byte
+    range: within 1e-4 of the CPU oracle.  Weights N(0, 1/n), so sums of order 1; at most
+    131072 terms meet in one running value (32 of the oracle's, 64 here), whose roundings add
+    up to about sqrt(131072) 2^-24 = 2.2e-5 of it."""
+    ff = (1 << 22) + 4
+    cfg = Config("llama", 8, ff, 1, 1, 1, 16, 40, rms_eps=1e-5, rope_theta=10000.0, tie_embeddings=True)
+    w = random_weights(cfg, seed=t, std=0.3)
+    w["layers"][0]["w_down"] *= np.float32(ff ** -0.5 / 0.3)
+    toks = [int(x) for x in random_prompt(t, t, cfg.vocab)]
+    om = ol.OracleModel(cfg, w)
+    want = om.forward(om.new_state(t), toks, all_logits=True)
+    with DeviceModel(cfg, w) as m:
+        got = m.forward(m.new_cache(t), toks, all_logits=True)
+    assert np.abs(got - want).max() < 1e-4
+
+
 @pytest.mark.parametrize("heads,kvh,n", [(9, 3, 100), (14, 2, 260), (3, 1, 500), (16, 2, 1000), (36, 2, 130)])
 def test_o_product_merges_the_chunks(heads, kvh, n):
     """Single-token steps over 2 to 17 chunks of 64 positions, whose states the o product

@@ -1104,8 +1104,7 @@ hipError_t gemm_epi(const GemmArgs &a, hipStream_t s) {
 
 hipError_t launch_gemm(int epi, const GemmArgs &a, hipStream_t s) {
     if (a.rows <= 0 || a.t <= 0) return hipSuccess;
-    // 80 rows of a tile within a signed 32-bit byte range
-    if (a.cols % 4 != 0 || a.cols > (1 << 22) || a.norm) return hipErrorInvalidValue;
+    if (a.cols % 4 != 0 || a.cols > kGemmCols || a.norm) return hipErrorInvalidValue;
     switch (epi) {
     case kEpiStore: return gemm_epi<kEpiStore>(a, s);
     case kEpiResid: return gemm_epi<kEpiResid>(a, s);

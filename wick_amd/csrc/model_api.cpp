@@ -185,8 +185,13 @@ int check_cache(const wick_hip_model *m, const wick_hip_kv *kv, int start, int t
 // Several tokens run their products on the matrix cores (gemm_kernel), except 2 or
 // 3 of a small model, which stream the weights through gemv_kernel in one pass:
 // the whole forward took 0.91 / 0.97 ms against 0.96 / 0.96 ms at hidden 576, but
-// 298 / 275 us against 259 / 235 us at hidden 2048.
-bool products_on_mfma(const wick_hip_model_config &c, int t) { return t >= 4 || (t > 1 && c.hidden > 1024); }
+// 298 / 275 us against 259 / 235 us at hidden 2048.  Rows past gemm_kernel's 32-bit
+// offsets take gemv_kernel, 4 tokens a pass.
+bool products_on_mfma(const wick_hip_model *m, int t) {
+    const wick_hip_model_config &c = m->c;
+    if (std::max({c.hidden, m->qd, c.intermediate}) > wick::kGemmCols) return false;
+    return t >= 4 || (t > 1 && c.hidden > 1024);
+}
 
 // One product with a fused epilogue: g.norm (optional) is the RMSNorm a GEMV
 // applies to its input rows; the GEMM takes it split (GemmArgs::ssq).
@@ -212,7 +217,7 @@ int forward_device(wick_hip_model *m, wick_hip_kv *kv, const uint32_t *tok_dev, 
     // embedding, the o and down products) also writes x * norm weight to xg and
     // its sums of squares to ssq, and the product that reads xg applies the
     // factor -- so no pass of its own reads x.
-    const bool gemm = products_on_mfma(c, t);
+    const bool gemm = products_on_mfma(m, t);
     int nssq = 1;
     if (!embedded) {
         hipError_t e = wick::launch_embed(m->embed, tok_dev, m->x, t, c.hidden, s, counters, gemm ? m->xg : nullptr,

@@ -85,7 +85,9 @@ hipError_t launch_gemv(int epi, const GemvArgs &a, hipStream_t s);
 hipError_t launch_gemv_states(const GemvArgs &a, const DecodeStates &st, hipStream_t s);
 
 // The same products for several tokens on the matrix cores (a.norm must be
-// null; kEpiQkv: splits and rows multiples of 16).
+// null; kEpiQkv: splits and rows multiples of 16); cols <= kGemmCols, so that the
+// 80 rows of its largest tile lie within a signed 32-bit byte range.
+constexpr int kGemmCols = 1 << 22;
 hipError_t launch_gemm(int epi, const GemmArgs &a, hipStream_t s);
 
 // x[i][:] = embed[tokens[i]][:] for i < t (token ids already validated).
