@@ -556,6 +556,31 @@ def test_prefill_split_over_workgroups(t, start, heads, kv_heads, d):
     assert within_tol(split, unsplit)[0]
 
 
+@pytest.mark.parametrize("t,start,heads,kv_heads,d,splits", [
+    (64, 832, 8, 8, 64, 3),      # 32 blocks, 7 steps
+    (64, 1088, 32, 4, 64, 1),    # 128 blocks, 9 steps: two splits would lose
+    (64, 1089, 32, 4, 64, 2),    # 10 steps
+    (192, 960, 8, 8, 64, 1),     # 96 blocks, 9 steps
+    (64, 512, 32, 8, 128, 1),    # 128 blocks, 9 steps at head_dim 128
+    (64, 513, 32, 8, 128, 2),    # 10 steps
+    (48, 336, 16, 8, 128, 3),    # 48 blocks, 6 steps
+    (48, 272, 16, 8, 128, 1),    # 5 steps
+])
+def test_prefill_split_rule(t, start, heads, kv_heads, d, splits):
+    """Where splitting starts to pay, by the workgroups a call launches (a split call's are
+    a multiple of its blocks)."""
+    import torch
+    with DeviceKvCache(1, start + t, kv_heads, d) as kv:
+        q = torch.zeros(t, heads * d, device="cuda")
+        att = torch.full_like(q, float("nan"))
+        torch.cuda.synchronize()
+        kv.attention_device(0, heads, q.data_ptr(), t, start, att.data_ptr())
+        kv.synchronize()
+        blocks = kv_heads * ((t * heads // kv_heads + 15) // 16)
+        assert kv.last_grid() == blocks * splits
+        assert att.eq(0).all()
+
+
 def test_prefill_split_calls_on_several_streams():
     """Split prefill calls of one handle on six streams at once, and replays of a captured
     call next to them: each stream's states are its own (the first four split, the others

@@ -1869,13 +1869,18 @@ int prefill_splits(int head_dim, int num_cus, const PrefillArgs &a) {
     const int steps = (a.start + a.t + 64 * tg - 1) / (64 * tg);  // of a wave of the last block, unsplit
     // Where half the CUs or more have a workgroup a split gains little or loses
     // (256 workgroups: 87 -> 107 us; 128: 46 -> 40), and below 6 steps the
-    // second launch costs what it saves (4 steps: 9.6 -> 10.3 us; 7: 12.6 ->
-    // 8.7).
+    // second launch costs what it saves (4 steps: 9.6 -> 10.3 us; 6, three splits
+    // of 16 blocks: 10.7 -> 9.9).
     if (2 * units > num_cus || steps < 6) return 1;
     // One workgroup per CU; two where that leaves a wave more than 8 steps (34
     // units of 94 steps: 27.6 -> 26.2 us; 32 of 63: 20.9, two 22.7).
     long long s = num_cus / units;
     if (steps > 8 * s) s = 2 * num_cus / units;
+    // Two splits halve the steps, where more of them take off two thirds: they pay
+    // from 10 steps (128 blocks at head_dim 128: 7 steps 12.4 -> 13.8 us, 9 14.7 ->
+    // 14.9, 10 15.8 -> 15.0; at 64: 7 11.9 -> 13.0, 8 12.9 -> 12.8 or, from other
+    // start positions, 12.3 -> 12.8, 10 15.3 -> 14.0).
+    if (s == 2 && steps < 10) return 1;
     return (int)std::max(1LL, std::min({s, steps / 2LL, kPrefillSplitGrid / units, (long long)kDecodeMaxChunks}));
 }
 
