@@ -95,12 +95,13 @@ def test_sampler_matches_oracle(vocab, name):
         assert ds.rng_state() == os_.rng.state()
 
 
-@pytest.mark.parametrize("vocab,top_k", [(4097, 2049), (4097, 0), (8192, 8191), (20001, 1025), (200003, 0)])
+@pytest.mark.parametrize("vocab,top_k", [(4097, 2049), (4097, 0), (8192, 8191), (20001, 1025), (200003, 0),
+                                         (99999, 2048), (99999, 2049), (100000, 1600), (100000, 1601)])
 def test_sort_over_many_workgroups(vocab, top_k):
     """Candidate sets sorted by several workgroups: the fewest ids that take that path, whole
-    and ragged tiles, one id left out, the smallest top-k that does; with infinite, NaN
-    (both signs) and equal logits, sums that never reach top-p, and a temperature at which
-    most terms vanish."""
+    and ragged tiles, one id left out, the smallest top-k that does and the largest that one
+    workgroup serves; with infinite, NaN (both signs) and equal logits, sums that never reach
+    top-p, and a temperature at which most terms vanish."""
     rng = np.random.default_rng(vocab + top_k)
     for cfg in (SamplerConfig(temperature=0.9, top_k=top_k, top_p=0.9, seed=3),
                 SamplerConfig(temperature=0.05, top_k=top_k, top_p=1.0, min_p=1e-6, seed=4),

@@ -1244,13 +1244,17 @@ hipError_t launch_sorted(const SampleArgs &a, hipStream_t s) {
 }  // namespace
 
 // Draws that launch_sorted serves: more candidates than one workgroup selects
-// and sorts faster, which takes about 18 us + k/32 + vocab/10000 against 55-65
-// us + vocab/5000 (151936 ids: k 200 44 against 70 us, 1000 71 / 71, 2000 107 /
-// 76, all of them 2288 / 96; 20000 ids: k 1000 50 / 63, 2000 77 / 64; 5000 ids:
-// k 2000 53 / 58, 4000 92 / 59).  Up to kList ids every set fits its LDS.
+// and sorts faster.  The workgroup's time steps up where its sort goes from 1024
+// to 2048 slots, at a k that depends on the logits (those that share their high
+// bits latest).  One workgroup against the sort, top-p 0.9: 20000 ids, k 1025 46
+// / 62 us, 1600 52 / 61, 2049 72 / 62, all of them 341 / 68; 32000 ids, k 1800,
+// logits of one exponent, 76 / 85; 65536, the same, 82 / 84, k 2048 103 / 81;
+// 100000 ids, the same, k 1400 78 / 84, 1600 99 / 88; 151936 ids, k 1025 69 / 74,
+// 1600 98 / 75, all of them 2267 / 101; 16384 ids, k 2049 73 / 64.  Up to kList
+// ids every set fits the workgroup's LDS.
 bool sorts_vocabulary(const SampleArgs &a) {
     const uint32_t k = top_k_of(a);
-    return !(a.temperature <= 0.0f) && a.vocab > kList && k > (a.vocab > 16384 ? 1024u : 2048u);
+    return !(a.temperature <= 0.0f) && a.vocab > kList && k > (a.vocab >= 100000 ? 1600u : 2048u);
 }
 
 hipError_t launch_sample(const SampleArgs &a, hipStream_t s) {
