@@ -45,6 +45,9 @@ constexpr int kList = 4096;            // largest candidate set sorted in LDS
 constexpr int kSlicePer = kSliceMax / kT;  // slice entries per thread in the split kernel
 constexpr int kPartCand = 1024;        // candidates one slice may hold at its k-th key
 constexpr int kQuickCand = 256;        // candidates placed by rank behind quick_bound; past these a radix select is cheaper
+// the slices' merge: past these one slice's k-th best is tried as the bound (logits
+// sorted by id, 49152 of them: k 40 21.6 -> 18.5 us, k 20 19.0 -> 17.1)
+constexpr int kOneCand = 192;
 
 typedef float f4 __attribute__((ext_vector_type(4)));
 
@@ -668,7 +671,17 @@ __global__ __launch_bounds__(kT) void sample_kernel(SampleArgs a) {
         uint32_t bound = ~wave_min(~b);
         if (have && (uint32_t)(mine >> 32) <= bound) s.l.cand[atomicAdd(&s.count, 1u)] = mine;
         __syncthreads();
-        if (s.count > (uint32_t)kQuickCand) {  // a few slices hold the best ids
+        if (s.count > (uint32_t)kOneCand) {  // a few slices hold the best ids: up to one's own k-th best
+            b = 0xffffffffu;
+            if (lane < a.parts && (int)k <= s.pcount[lane]) b = (uint32_t)(a.part_cand[lane * kFastK + k - 1] >> 32);
+            bound = wave_min(b);
+            __syncthreads();
+            if (tid == 0) s.count = 0u;
+            __syncthreads();
+            if (have && (uint32_t)(mine >> 32) <= bound) s.l.cand[atomicAdd(&s.count, 1u)] = mine;
+            __syncthreads();
+        }
+        if (s.count > (uint32_t)kQuickCand) {  // hundreds of equal ids
             const uint32_t total = (uint32_t)__syncthreads_count(have);
             bound = 0xffffffffu;
             if (k < total)
