@@ -554,18 +554,23 @@ def test_o_product_merges_the_chunks(heads, kvh, n):
         assert [first] + m.decode(cache, first, 59) == ids
 
 
-@pytest.mark.parametrize("hidden,ff,vocab", [
-    (2052, 2050 * 4, 2100),   # every product on the long-row kernel: 4 columns past a pass, rows left over
-    (2304, 14336, 4099),      # its longest row, a head whose last pair is short
-    (2304, 14340, 2048),      # one past it
-    (4096, 1028, 1024),       # whole passes; a down product too narrow for it
+@pytest.mark.parametrize("hidden,ff,vocab,heads", [
+    # on the kernel for long rows (model.hip, gemv_wide):
+    (2052, 2050 * 4, 2100, 4),   # gate/up, 4 columns past a pass, rows left over
+    (2304, 14336, 4099, 4),      # gate/up, and a head whose last pair is short
+    (2304, 14340, 2048, 4),      # gate/up; a down product of rows one past its longest
+    (4096, 1028, 1024, 4),       # gate/up in whole passes, the fewest weights
+    (3076, 12292, 4100, 20),     # every product, the shortest rows and fewest rows of a down product
+    (4096, 14336, 14336, 14),    # every product: its longest row, the most rows of a down product,
+                                 # q/k/v rows and a head's rounds just long enough
+    (4100, 2056, 14332, 4),      # none: gate/up just past 2048 rows, a head one pair short of its rounds
 ])
-def test_single_token_products_on_long_rows(hidden, ff, vocab):
-    """One-token forwards whose rows are too long for one pass: logits of 4 steps within 1e-4
-    of the CPU oracle and the same greedy ids.  Weights N(0, 1/hidden), so products of unit-rms
-    rows are of order 1 and two orders of a sum of n terms differ by about sqrt(n) 2^-24,
-    at most 8e-6 here."""
-    cfg = Config("llama", hidden, ff, 1, 4, 2, 64, vocab, rms_eps=1e-5, rope_theta=10000.0, tie_embeddings=True)
+def test_single_token_products_on_long_rows(hidden, ff, vocab, heads):
+    """One-token forwards whose rows are too long for one pass: logits of 4 steps, as the last
+    token's and as all tokens', within 1e-4 of the CPU oracle and the same greedy ids.
+    Weights N(0, 1/hidden), so products of unit-rms rows are of order 1 and two orders of a sum
+    of n terms differ by about sqrt(n) 2^-24, at most 8e-6 here."""
+    cfg = Config("llama", hidden, ff, 1, heads, 2, 64, vocab, rms_eps=1e-5, rope_theta=10000.0, tie_embeddings=True)
     w = random_weights(cfg, seed=hidden, std=hidden ** -0.5)
     rng = np.random.default_rng(ff)
     w["norm"] = (1 + 0.2 * rng.standard_normal(hidden)).astype(np.float32)
@@ -578,6 +583,9 @@ def test_single_token_products_on_long_rows(hidden, ff, vocab):
         for _ in range(4):
             want = om.forward(st, [tok])
             got = m.forward(cache, [tok])
+            assert np.abs(got - want).max() < 1e-4
+            cache.len -= 1
+            got = m.forward(cache, [tok], all_logits=True)
             assert np.abs(got - want).max() < 1e-4
             tok = ol.argmax(want[0])
             ids.append(tok)

@@ -953,13 +953,31 @@ hipError_t gemv1_launch(const GemvArgs &a, hipStream_t s) {
     return hipErrorInvalidValue;
 }
 
-// Where gemv_wide_kernel is the faster one: 16 MB of weights or more (the head
-// at 1001 x 2052: 7.9 against 9.3 us), the row (padded to passes of 2048 columns)
-// and the waves' sums within 64 KiB of LDS, and either a norm (gemv_kernel then
-// reads the input row twice) or rows of 8192 columns and more (2048 x 5632: 9.6
-// against 9.9 us; 4096 x 4096 equal).
+// Where gemv_wide_kernel is the faster one: 16 MB of weights or more, and the row
+// (padded to passes of 2048 columns) and the waves' sums within 64 KiB of LDS.
+// Its workgroups of 8 waves fill the CUs in coarser steps than gemv_kernel's 4, so
+// past that the lines lie where its rounds are full (weights not in cache, us):
+//   o / down (no norm): rows of 12288 columns and more, over three quarters to one
+//     round of 512 workgroups (3716 x 14336 40.6 -> 36.7, 4096 x 14336 40.1 -> 39.3;
+//     3072 x 14336 31.1 against 32.1, 4612 x 12288 40.9 / 42.1, 8192 columns 13.5 / 14.7)
+//   gate/up: not from 2048 to 3072 rows (2436 x 3072 16.4 / 17.1), nor rows a multiple
+//     of 32 KB apart (8192 x 8192 96.1 / 101.2); else 5 to 40% faster
+//   the head: more than 4096 rows, and past 8192 rounds of 8192 rows at least seven
+//     eighths full, up to 8 of them (4228 x 4096 23.3 -> 20.3, 32000 x 4096 104 -> 98;
+//     3072 x 3072 13.2 / 13.9, 10244 x 4096 37.7 / 40.8, 20484 x 3072 43.7 / 45.5,
+//     128256 x 3072 238 / 244)
+//   q/k/v: always (5 to 60% faster).
+template <int EPI>
 bool gemv_wide(const GemvArgs &a) {
-    return (long long)a.rows * a.cols >= (4 << 20) && a.cols <= 7 * 2048 && (a.norm ? a.cols > 2048 : a.cols >= 8192);
+    if ((long long)a.rows * a.cols < (4 << 20) || a.cols > 7 * 2048) return false;
+    if (EPI == kEpiResid) return !a.norm && a.cols >= 12288 && a.rows > 3072 && a.rows <= 4096;
+    if (!a.norm || a.cols <= 2048) return false;
+    if (EPI == kEpiSwiglu) return a.cols % 8192 != 0 && (a.rows <= 2048 || a.rows > 3072);
+    if (EPI == kEpiStore || EPI == kEpiArgmax) {
+        const long long rounds = (a.rows + 8191LL) / 8192;
+        return a.rows > 4096 && rounds <= 8 && (rounds == 1 || 8LL * a.rows >= 7 * 8192 * rounds);
+    }
+    return true;
 }
 
 template <int R, int U, int EPI>
@@ -967,10 +985,7 @@ hipError_t gemv_wide_launch(const GemvArgs &a, hipStream_t s) {
     const int groups = (a.rows + R - 1) / R, passes = ((a.cols >> 2) + 64 * U - 1) / (64 * U);
     const dim3 grid((unsigned)std::min((groups + kWideWaves - 1) / kWideWaves, 512)), block(64 * kWideWaves);
     const size_t lds = (size_t)passes * 64 * U * sizeof(f4);
-    if (a.norm)
-        hipLaunchKernelGGL((gemv_wide_kernel<R, U, EPI, true>), grid, block, lds, s, a);
-    else
-        hipLaunchKernelGGL((gemv_wide_kernel<R, U, EPI, false>), grid, block, lds, s, a);
+    hipLaunchKernelGGL((gemv_wide_kernel<R, U, EPI, EPI != kEpiResid>), grid, block, lds, s, a);
     return hipGetLastError();
 }
 
@@ -984,16 +999,16 @@ hipError_t gemv_epi(const GemvArgs &a, hipStream_t s) {
     if constexpr (EPI == kEpiArgmax) {
         if (a.t != 1 || !a.out1) return hipErrorInvalidValue;
         if (a.cols <= 4 * 64 * 4) return gemv1_launch<kArgmaxRows, EPI>(a, s);
-        if (gemv_wide(a)) return gemv_wide_launch<kArgmaxRows, 2, EPI>(a, s);
+        if (gemv_wide<EPI>(a)) return gemv_wide_launch<kArgmaxRows, 2, EPI>(a, s);
         return gemv_launch<1, kArgmaxRows, 4, EPI>(a, s);
     } else {
         if (a.t > 1) return gemv_launch<4, 1, 4, EPI>(a, s);
         if constexpr (EPI == kEpiStore) {
             if (a.cols <= 4 * 64 * 4) return gemv1_launch<4, EPI>(a, s);
-            if (gemv_wide(a)) return gemv_wide_launch<4, 2, EPI>(a, s);
+            if (gemv_wide<EPI>(a)) return gemv_wide_launch<4, 2, EPI>(a, s);
             return gemv_launch<1, 4, 4, EPI>(a, s);
         }
-        if (gemv_wide(a)) return gemv_wide_launch<1, EPI == kEpiSwiglu ? 4 : 8, EPI>(a, s);
+        if (gemv_wide<EPI>(a)) return gemv_wide_launch<1, EPI == kEpiSwiglu ? 4 : 8, EPI>(a, s);
         if (one_pass) return gemv1_launch<1, EPI>(a, s);
         return gemv_launch<1, 1, 8, EPI>(a, s);
     }
