@@ -520,10 +520,12 @@ def test_decode_hip_graph_replays_match_eager():
     (3, 700, 6, 6, 128),      # one head per kv head, 3 rows
     (64, 1984, 32, 4, 64),    # 128 blocks: the most that split
     (2, 70000, 8, 1, 64),     # as many splits as states can be merged
+    (2048, 0, 1, 1, 64),      # a whole prompt: the first block has one tile of keys for two splits
+    (1500, 3, 1, 1, 128),     # ... and for five
 ])
 def test_prefill_split_over_workgroups(t, start, heads, kv_heads, d):
-    """A few tokens over many keys: the blocks' keys shared by several workgroups and
-    merged, against the oracle and against the entry point that never splits; bit-stable;
+    """A few blocks over many keys: the blocks' keys shared by several workgroups and
+    merged, some of which a short block leaves without keys, against the oracle and against the entry point that never splits; bit-stable;
     and unsplit, without allocating, where the call is captured into a graph."""
     import torch
     q, k, v = make_inputs(start, t, start, heads, kv_heads, d, theta=1e6)

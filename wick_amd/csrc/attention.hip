@@ -1477,9 +1477,9 @@ __device__ __forceinline__ void prefill_lean_body(const PrefillArgs &a) {
             for (int rr = 0; rr < 4; rr++) sm_o[w][16 * rb + col][out_dim<D>(g, rr, db)] = o[rb][db][rr];
     }
     __syncthreads();
-    // Merge the 4 waves' states (log2 units); wave 0 holds key 0, so M is
-    // finite (a wave or split without keys keeps the finite floor and l = 0).
-    // The per-column weights, 1/sum and output row come first, once per column,
+    // Merge the 4 waves' states (log2 units).  M is finite: a wave without keys
+    // keeps the finite floor, l = 0 and o = 0, and so does the state of a split
+    // without any (a block of fewer tiles than splits has such).  The per-column weights, 1/sum and output row come first, once per column,
     // so the per-element pass is 4 LDS float4 reads and FMAs.  A split's merged
     // state goes to the workspace, unnormalised, at [row][split].
     if (threadIdx.x < R) {
