@@ -474,19 +474,33 @@ def test_random_config_sweep(case):
     assert got == want
 
 
-@pytest.mark.parametrize("hidden,ff,vocab,t", [
-    (36, 20, 37, 4),       # 16-token tiles: rows and columns that fill no block or k-step
-    (2052, 36, 40, 16),    # ... with the deep batches of 2048 columns and more
-    (64, 1028, 300, 17),   # 32-token tiles, 15 tokens of the second block missing
-    (36, 4112, 2045, 251),  # gate/up on 2 x 2 blocks, the LM head on 2 x 4
-    (4108, 20, 300, 33),   # o and down products on 2 x 2 blocks, a 12-row last block
-    (36, 20, 2557, 251),   # the LM head on 5 x 2 blocks, a row count that is no multiple of 4
-])
-def test_products_of_several_tokens(hidden, ff, vocab, t):
-    """Every tile of the matrix-core products and their edges: all t rows of logits, alone
-    and after 3 cached tokens (fewer than the matrix cores take at this width), within 1e-4
-    of the CPU oracle (the bound for another summation order)."""
-    cfg = Config("llama", hidden, ff, 2, 2, 1, 16, vocab, rms_eps=1e-5, rope_theta=10000.0, tie_embeddings=True)
+# hidden, ff, query heads, kv heads, head_dim, vocabulary, tokens.  What each is there for
+# names the tiles as 16-row blocks x 16-token blocks; test_gemm_tiles.py checks that every
+# tile is among them in each epilogue.
+PRODUCT_CASES = [
+    (36, 20, 2, 1, 16, 37, 4),          # 1x1: rows and columns that fill no block or k-step
+    (2052, 36, 2, 1, 16, 40, 16),       # ... with the deep batches of 2048 columns and more
+    (580, 2052, 16, 1, 16, 37, 4),      # ... on 8 waves; a deep down product, rows over by 4
+    (64, 1028, 2, 1, 16, 300, 17),      # 1x2, 15 tokens of the second block missing
+    (36, 4112, 2, 1, 16, 2045, 251),    # gate/up of 257 row blocks, the LM head on 2x4
+    (4108, 20, 2, 1, 16, 300, 33),      # o and down products of a 12-row last block
+    (36, 20, 2, 1, 16, 2557, 251),      # the LM head on 5x2, a row count that is no multiple of 4
+    (580, 20, 8, 1, 64, 700, 200),      # q/k/v, o, down and the LM head on 2x2, a last tile of 4
+                                        # rows, 8 tokens
+    (164, 20, 40, 1, 64, 2557, 33),     # q/k/v and the LM head on 2x2 and 6 waves
+    (292, 36, 48, 1, 64, 37, 100),      # q/k/v on 2x4, a last tile of 36 tokens
+    (260, 20, 48, 2, 64, 300, 130),     # q/k/v on 5x2, a last tile of 3 blocks, 2 tokens
+    (1604, 292, 1, 1, 16, 37, 251),     # o and down on 2x4, a last tile of 4 rows, 59 tokens
+    (2564, 516, 1, 1, 16, 37, 200),     # o and down on 5x2, a last tile of 4 rows, 8 tokens
+]
+
+
+@pytest.mark.parametrize("hidden,ff,heads,kvh,d,vocab,t", PRODUCT_CASES)
+def test_products_of_several_tokens(hidden, ff, heads, kvh, d, vocab, t):
+    """Every tile of the matrix-core products in every epilogue, and their edges: all t rows
+    of logits, alone and after 3 cached tokens (fewer than the matrix cores take up to 1024
+    columns), within 1e-4 of the CPU oracle (the bound for another summation order)."""
+    cfg = Config("llama", hidden, ff, 2, heads, kvh, d, vocab, rms_eps=1e-5, rope_theta=10000.0, tie_embeddings=True)
     w = random_weights(cfg, seed=hidden + t, std=hidden ** -0.5)
     rng = np.random.default_rng(hidden)
     w["norm"] = (1 + 0.2 * rng.standard_normal(hidden)).astype(np.float32)

@@ -15,6 +15,7 @@
 
 #include <algorithm>
 
+#include "gemm_tiles.h"
 #include "model_kernels.h"
 #include "wave_ops.h"
 
@@ -1067,52 +1068,26 @@ hipError_t gemm_launch(const GemmArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// 8 waves, or 6 where those take no more batches of 32 columns each (576 columns
-// are 18: 3 either way; 16 tokens of gate/up 6.2 against 6.5 us, 251 tokens of o
-// 6.3 against 6.5; where they take more, up to a quarter slower).
-template <int EPI, int RB, int TB>
-hipError_t gemm_waves(const GemmArgs &a, hipStream_t s) {
-    const int nbat = (a.cols + 31) / 32;
-    if ((nbat + 5) / 6 == (nbat + 7) / 8) return gemm_launch<EPI, RB, TB, 6, 2>(a, s);
-    return gemm_launch<EPI, RB, TB, 8, 2>(a, s);
-}
-
-// What a tile of rb x tb blocks costs: the products of the busiest of the 256
-// CUs, each dearer the less the tile reuses what it loads.  The model's order
-// is the measured one where the tiles differ by more than a few percent: 64
-// tokens at 2048 x 2048: 1x2 10 us, 2x2 12.6; 251 tokens at 2560 x 2048: 5x2
-// 27.5, 1x2 30.2, 2x2 30.7; at 2048 x 5632: 2x4 47.3, 2x2 50.4; at 576 x 576:
-// 2x2 6.3, 1x2 6.6, 2x4 8.
-double gemm_cost(const GemmArgs &a, int rb, int tb) {
-    const long long wgs = (long long)((a.rows + 16 * rb - 1) / (16 * rb)) * ((a.t + 16 * tb - 1) / (16 * tb));
-    return (double)((wgs + 255) / 256) * (rb * tb + 0.5 * (rb + tb));
-}
-
 template <int EPI>
 hipError_t gemm_epi(const GemmArgs &a, hipStream_t s) {
-    if (a.t <= 16) {
-        // bound by the weights' arrival: more of them in flight per wave where a
-        // wave takes several batches (4 tokens, 2048 x 5632: 13.7 against 17.4
-        // us; at 576 columns a batch of 4 leaves waves idle, 4.1 against 3.5)
-        if constexpr (EPI != kEpiSwiglu)
-            if (a.cols >= 2048) return gemm_launch<EPI, 1, 1, 8, 4>(a, s);
-        return gemm_waves<EPI, 1, 1>(a, s);
-    }
+    const GemmTile x = gemm_tile(EPI == kEpiSwiglu, a.rows, a.cols, a.t);
+    const auto is = [&](int rb, int tb, int waves, int ku) {
+        return x.rb == rb && x.tb == tb && x.waves == waves && x.ku == ku;
+    };
+    if (is(1, 1, 6, 2)) return gemm_launch<EPI, 1, 1, 6, 2>(a, s);
+    if (is(1, 1, 8, 2)) return gemm_launch<EPI, 1, 1, 8, 2>(a, s);
+    if (is(1, 2, 8, 2)) return gemm_launch<EPI, 1, 2, 8, 2>(a, s);
     if constexpr (EPI == kEpiSwiglu) {
-        // Larger tiles of both matrices fill a CU's LDS with one workgroup: 251
-        // tokens at 5632 x 2048 114 us on 2x2 against 110.  8 waves leave room
-        // for two, worth it where a wave takes many batches (at 1536 x 576 21
-        // against 14.1 us on 4 waves; at 5632 x 2048 110 against 118).
-        return a.cols < 1024 ? gemm_launch<EPI, 1, 2, 4, 2>(a, s) : gemm_launch<EPI, 1, 2, 8, 2>(a, s);
+        if (is(1, 2, 4, 2)) return gemm_launch<EPI, 1, 2, 4, 2>(a, s);
     } else {
-        const int tiles[][2] = {{1, 2}, {2, 2}, {2, 4}, {5, 2}};
-        int best = 0;
-        for (int i = 1; i < 4; i++)
-            if (gemm_cost(a, tiles[i][0], tiles[i][1]) < gemm_cost(a, tiles[best][0], tiles[best][1])) best = i;
-        if (best == 3) return gemm_launch<EPI, 5, 2, 8, 2>(a, s);
-        if (best == 2) return gemm_launch<EPI, 2, 4, 8, 2>(a, s);
-        return best == 1 ? gemm_waves<EPI, 2, 2>(a, s) : gemm_waves<EPI, 1, 2>(a, s);
+        if (is(1, 1, 8, 4)) return gemm_launch<EPI, 1, 1, 8, 4>(a, s);
+        if (is(1, 2, 6, 2)) return gemm_launch<EPI, 1, 2, 6, 2>(a, s);
+        if (is(2, 2, 6, 2)) return gemm_launch<EPI, 2, 2, 6, 2>(a, s);
+        if (is(2, 2, 8, 2)) return gemm_launch<EPI, 2, 2, 8, 2>(a, s);
+        if (is(2, 4, 8, 2)) return gemm_launch<EPI, 2, 4, 8, 2>(a, s);
+        if (is(5, 2, 8, 2)) return gemm_launch<EPI, 5, 2, 8, 2>(a, s);
     }
+    return hipErrorInvalidValue;
 }
 
 }  // namespace
