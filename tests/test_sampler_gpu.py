@@ -139,12 +139,13 @@ def test_draw_that_starts_from_zero(vocab, top_p):
         assert ds.rng_state() == os_.rng.state()
 
 
-@pytest.mark.parametrize("vocab,top_k", [(70, 64), (4096, 40), (4097, 64), (16384, 64), (49152, 1), (49152, 40), (65537, 16),
-                                         (65537, 17), (196608, 64)])
+@pytest.mark.parametrize("vocab,top_k", [(70, 64), (4096, 40), (4097, 64), (16384, 64), (49152, 1), (49152, 40),
+                                         (65537, 16), (65537, 17), (196608, 64)])
 def test_top_k_behind_a_loose_bound(vocab, top_k):
     """The top-k taken per slice behind a bound from its waves, then from the slices, or from
-    one of them: one and two ids a wave, a slice of two ids, the longest slices; and logits whose bound is loose
-    (the best ids all in one slice or in one wave, hundreds of equal ones), infinite and NaN."""
+    one of them: one and two ids a wave, a slice of two ids, the longest slices; and logits
+    whose bound is loose (the best ids all in one slice or in one wave, hundreds of equal
+    ones), infinite and NaN."""
     rng = np.random.default_rng(vocab + top_k)
     cfg = SamplerConfig(temperature=0.9, top_k=top_k, top_p=0.95, seed=3)
     with DeviceSampler(cfg, vocab) as ds:

@@ -1553,8 +1553,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void p
 // all keys, at about 1.35 us a step.  The key range is split again over
 // a.splits workgroups (prefill_splits), each writing its rows' states, and
 // prefill_merge_kernel, the next launch (3.5 us), combines them.  37 tokens on
-// 12001 positions, Qwen2.5 shape: 124 -> 26 us (34 workgroups -> 510); 5
-// tokens 124 -> 12; 16 on 8000, Llama-3-8B shape: 181 -> 34.  Two row blocks
+// 12001 positions, Qwen2.5 shape: 122 -> 24 us (34 workgroups -> 510); 5
+// tokens 124 -> 11; 16 on 8000, Llama-3-8B shape: 156 -> 28.  Two row blocks
 // per workgroup gain nothing here (29 us for the first).
 template <int D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 128 ? 3 : 4)))

@@ -38,9 +38,11 @@ inline GemmTile gemm_tile(bool gate_up, int rows, int cols, int t) {
         return {1, 1, gemm_waves(cols), 2};
     }
     // Larger tiles of both matrices fill a CU's LDS with one workgroup: 251
-    // tokens at 5632 x 2048 114 us on 2x2 against 110.  8 waves leave room
-    // for two, worth it where a wave takes many batches (at 1536 x 576 21
-    // against 14.1 us on 4 waves; at 5632 x 2048 110 against 118).
+    // tokens at 5632 x 2048 114 us on 2x2 against 110.  8 waves leave room for
+    // two; with 4 more workgroups fit where a wave takes few batches.  251 tokens
+    // on 4 / 8 waves: 1536 x 576 13.6 / 20.7 us, 4864 x 896 47 / 59, 5632 x 2048
+    // 111 / 109.  Between, a few tokens want 8 and many want 4: 17 and 251 tokens at
+    // 3072 x 1024 11.3 / 10.8 and 36 / 38, at 3456 x 1280 14.1 / 12.6 and 46 / 53.
     if (gate_up) return {1, 2, cols < 1024 ? 4 : 8, 2};
     const int tiles[][2] = {{1, 2}, {2, 2}, {2, 4}, {5, 2}};
     int best = 0;

@@ -183,9 +183,11 @@ int check_cache(const wick_hip_model *m, const wick_hip_kv *kv, int start, int t
 }
 
 // Several tokens run their products on the matrix cores (gemm_kernel), except 2 or
-// 3 of a small model, which stream the weights through gemv_kernel in one pass:
-// the whole forward took 0.91 / 0.97 ms against 0.96 / 0.96 ms at hidden 576, but
-// 298 / 275 us against 259 / 235 us at hidden 2048.  Rows past gemm_kernel's 32-bit
+// 3 of a small model, which stream the weights through gemv_kernel in one pass.
+// Forwards of 2 / 3 tokens through 16 layers, gemv_kernel against the matrix cores:
+// hidden 576 559 / 572 us against 563 / 555, 896 762 / 795 against 750 / 738, 1024
+// (8 kv heads of 64) 663 / 706 against 680 / 670; through 4 layers, 1536 397 / 409
+// against 337 / 340.  Rows past gemm_kernel's 32-bit
 // offsets take gemv_kernel, 4 tokens a pass.
 bool products_on_mfma(const wick_hip_model *m, int t) {
     const wick_hip_model_config &c = m->c;
