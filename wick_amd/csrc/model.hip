@@ -525,7 +525,7 @@ __global__ __launch_bounds__(256) void gemv1_states_kernel(const GemvArgs a, con
 // length from L2.  In the MFMA lane layout consecutive lanes are consecutive
 // rows, and the L1 then serves one lane (16 bytes) a cycle: 65 cache accesses
 // per load instruction counted, 13 to 15 bytes per cycle and CU whatever the tile
-// (profiles/pmc_l1_products_tinyllama_256.md; 13 to 16 accesses in this layout).
+// (13 to 16 accesses as loaded here).
 // So a wave loads 16 rows x 32 k with 8 consecutive lanes on one row's 128-byte
 // line (4 lanes on 64 bytes: 5 to 20% slower) and passes it through its own
 // piece of LDS.  251 tokens of a 2048-wide layer (hidden 2048, FFN 5632): q/k/v
